@@ -8,6 +8,7 @@
 #include <cmath>
 #include <string>
 #include <mutex>
+#include <algorithm>
 #include <set>
 #include "fx_lbm.h"
 #include "lbm_launch.hpp"
@@ -48,6 +49,9 @@ struct fx_ctx {
 	double* result = nullptr;  // 4 doubles (device)
 	double* scratch = nullptr; // this device's copy of the static scratch array (fx_lbm_mass_sum_noalloc)
 	std::set<void*> buffers;   // allocations owned by this context
+	fx::TwoStepShape shape_two{}; // two_steps launches of fx_lbm_run and fx_lbm_forward
+	void* second = nullptr;    // DDF array that two_steps launches alternate with (SecondArray)
+	bool second_busy = false;  // a call is queueing launches on it
 };
 
 struct fx_adjoint {
@@ -97,14 +101,119 @@ int resolve_scratch(int device, double** out) {
 	return FX_OK;
 }
 
+uint64_t ddf_bytes(const fx_ctx* ctx) {
+	return ctx->N * (uint64_t)ctx->cfg.velocity_set * (ctx->cfg.storage == FX_FP32 ? 4u : 2u);
+}
+
+// ---- second DDF arrays ----
+// two_steps launches read one DDF array and write another.  The second one belongs to the
+// context that runs them and is allocated by its first run that can use it, if at least half
+// of the device memory stays free; it is kept for the next run, and given back when any
+// context of the device cannot allocate what its caller asked for (allocate_device), or with
+// the context.  Launches on one context's stream run in order, so the next call may use the
+// array while the last one's launches still run; a call from another thread that comes while
+// one is queueing takes single steps.  g_second_mutex guards the list and every context's
+// `second` and `second_busy`.
+std::mutex g_second_mutex;
+std::set<fx_ctx*> g_second_owners;
+
+// Allocations must not disturb a stream capture that another library has open in this thread.
+struct RelaxedCapture {
+	hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+	RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+	~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+void release_second_locked(fx_ctx* ctx) {
+	if(!ctx->second) return;
+	const RelaxedCapture relaxed;
+	(void)hipStreamSynchronize(ctx->stream);
+	(void)hipFree(ctx->second);
+	ctx->second = nullptr;
+	g_second_owners.erase(ctx);
+}
+// Gives back every second array of the device that no call is using; true if there was one.
+bool release_second_arrays(int device) {
+	std::lock_guard<std::mutex> lock(g_second_mutex);
+	bool any = false;
+	const std::set<fx_ctx*> owners = g_second_owners;
+	for(fx_ctx* c : owners)
+		if(c->device == device && !c->second_busy) { release_second_locked(c); any = true; }
+	return any;
+}
+hipError_t allocate_device(int device, void** p, uint64_t bytes) {
+	hipError_t e = hipMalloc(p, bytes);
+	if(e != hipSuccess && release_second_arrays(device)) {
+		(void)hipGetLastError();
+		e = hipMalloc(p, bytes);
+	}
+	return e;
+}
+// Free memory of the current device, counting second arrays that would be given back.
+hipError_t free_memory(int device, uint64_t need, uint64_t* free_bytes) {
+	size_t f = 0, total = 0;
+	hipError_t e = hipMemGetInfo(&f, &total);
+	if(e == hipSuccess && need > (uint64_t)f && release_second_arrays(device)) e = hipMemGetInfo(&f, &total);
+	*free_bytes = (uint64_t)f;
+	return e;
+}
 int ensure_partial(fx_ctx* ctx, uint64_t doubles) {
 	if(ctx->partial_cap >= doubles) return FX_OK;
 	if(ctx->partial) FX_HIP(hipFree(ctx->partial));
 	ctx->partial = nullptr;
 	ctx->partial_cap = 0;
-	FX_HIP(hipMalloc(&ctx->partial, doubles * sizeof(double)));
+	FX_HIP(allocate_device(ctx->device, (void**)&ctx->partial, doubles * sizeof(double)));
 	ctx->partial_cap = doubles;
 	return FX_OK;
+}
+
+// The context's second DDF array while the object lives (array == nullptr: there is none).
+struct SecondArray {
+	fx_ctx* ctx;
+	void* array = nullptr;
+	explicit SecondArray(fx_ctx* c) : ctx(c) {
+		std::lock_guard<std::mutex> lock(g_second_mutex);
+		if(ctx->second_busy) return; // another thread is queueing launches on it
+		if(!ctx->second) {
+			const RelaxedCapture relaxed;
+			size_t f = 0, total = 0;
+			if(hipMemGetInfo(&f, &total) != hipSuccess || ddf_bytes(ctx) + total / 2u > f) { (void)hipGetLastError(); return; }
+			if(hipMalloc(&ctx->second, ddf_bytes(ctx)) != hipSuccess) { (void)hipGetLastError(); ctx->second = nullptr; return; }
+			g_second_owners.insert(ctx);
+		}
+		ctx->second_busy = true;
+		array = ctx->second;
+	}
+	~SecondArray() {
+		if(!array) return;
+		std::lock_guard<std::mutex> lock(g_second_mutex);
+		ctx->second_busy = false;
+	}
+	SecondArray(const SecondArray&) = delete;
+	SecondArray& operator=(const SecondArray&) = delete;
+};
+
+// Queues steps t .. t+steps-1 on a.fi.  Pairs of two_steps launches, fi -> second -> fi, take
+// four steps each and leave the DDFs where they were; the rest are single steps.
+void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps) {
+	if(steps >= 4u && ctx->shape_two.grid) {
+		SecondArray second(ctx);
+		if(second.array) {
+			void* const fi = a.fi;
+			a.odd = (uint32_t)(t & 1ull);
+			for(; steps >= 4u; steps -= 4u, t += 4u) {
+				a.fi = fi;
+				ctx->k->two_steps(a, second.array, ctx->shape_two, ctx->stream);
+				a.fi = second.array;
+				ctx->k->two_steps(a, fi, ctx->shape_two, ctx->stream);
+			}
+			a.fi = fi;
+		}
+	}
+	for(; steps > 0u; steps--, t++) {
+		a.odd = (uint32_t)(t & 1ull);
+		ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+	}
 }
 
 fx::LbmArgs make_args(const fx_ctx* ctx, const void* fi, const float* rho, const float* u, const uint8_t* flags, uint64_t t,
@@ -473,13 +582,18 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	if(e == hipSuccess) {
 		hipDeviceProp_t prop;
 		e = hipGetDeviceProperties(&prop, device);
+		// k_two_steps has 32-bit byte offsets within a plane
+		if(e == hipSuccess && ctx->k->two_steps && (uint64_t)cfg->Nx * cfg->Ny * eb <= 0xFFFFFFFFull) {
+			const fx::TwoStepShape two = fx::two_step_shape(cfg->Nx, cfg->Ny, cfg->Nz, (uint32_t)prop.multiProcessorCount);
+			if(fx::two_steps_pay(two, cfg->Nx, cfg->Ny, cfg->Nz, cfg->velocity_set, cfg->collision == FX_TRT, cfg->extensions)) ctx->shape_two = two;
+		}
 		if(e == hipSuccess && cap)
 			ctx->shape_sc.lds = fx::occupancy_lds(cap, ctx->shape_sc.block.x, prop.maxSharedMemoryPerMultiProcessor, prop.sharedMemPerBlock);
 	}
 	if(e == hipSuccess) {
-		size_t free_b = 0, total_b = 0;
-		e = hipMemGetInfo(&free_b, &total_b);
-		if(e == hipSuccess && N * fx_memory_bytes_per_cell(cfg) > (uint64_t)free_b) {
+		uint64_t free_b = 0;
+		e = free_memory(device, N * fx_memory_bytes_per_cell(cfg), &free_b);
+		if(e == hipSuccess && N * fx_memory_bytes_per_cell(cfg) > free_b) {
 			delete ctx;
 			return fail(FX_ERR_MEMORY, "Grid resolution is too large for the free device memory");
 		}
@@ -487,7 +601,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	if(e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
 	if(e == hipSuccess) e = hipEventCreate(&ctx->ev0);
 	if(e == hipSuccess) e = hipEventCreate(&ctx->ev1);
-	if(e == hipSuccess) e = hipMalloc(&ctx->result, 4 * sizeof(double));
+	if(e == hipSuccess) e = allocate_device(device, (void**)&ctx->result, 4 * sizeof(double));
 	if(e != hipSuccess) {
 		fx_ctx_destroy(ctx);
 		return fail_hip(e, "fx_ctx_create");
@@ -505,6 +619,10 @@ int fx_ctx_destroy(fx_ctx* ctx) {
 	if(!ctx) return FX_OK;
 	(void)hipSetDevice(ctx->device);
 	if(ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+	{
+		std::lock_guard<std::mutex> lock(g_second_mutex);
+		release_second_locked(ctx);
+	}
 	for(void* p : ctx->buffers) (void)hipFree(p);
 	if(ctx->partial) (void)hipFree(ctx->partial);
 	if(ctx->result) (void)hipFree(ctx->result);
@@ -533,7 +651,7 @@ int fx_buf_alloc(fx_ctx* ctx, uint64_t bytes, void** dptr) {
 	if(bytes == 0ull) return fail(FX_ERR_ARG, "Memory size must be larger than 0");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
 	void* p = nullptr;
-	const hipError_t e = hipMalloc(&p, bytes);
+	const hipError_t e = allocate_device(ctx->device, &p, bytes);
 	if(e != hipSuccess) return fail(FX_ERR_MEMORY, std::string("hipMalloc of ") + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
 	ctx->buffers.insert(p);
 	*dptr = p;
@@ -621,16 +739,12 @@ int fx_lbm_run(fx_ctx* ctx, void* fi, float* rho, float* u, const uint8_t* flags
 	const int rc = check_step_args(ctx, fi, rho, u, flags, F, alpha);
 	if(rc != FX_OK) return rc;
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-	fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, t0, fx_, fy_, fz_, F, alpha);
-	for(uint64_t s = 0; s < steps; s++) {
-		a.odd = (uint32_t)((t0 + s) & 1ull);
-		ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
-	}
+	if(ms) FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+	queue_steps(ctx, make_args(ctx, fi, rho, u, flags, t0, fx_, fy_, fz_, F, alpha), t0, steps);
 	const int lc = check_launch("stream_collide");
 	if(lc != FX_OK) return lc;
-	FX_HIP(hipEventRecord(ctx->ev1, ctx->stream));
 	if(ms) {
+		FX_HIP(hipEventRecord(ctx->ev1, ctx->stream));
 		FX_HIP(hipEventSynchronize(ctx->ev1));
 		FX_HIP(hipEventElapsedTime(ms, ctx->ev0, ctx->ev1));
 	}
@@ -728,9 +842,6 @@ int fx_lbm_mass_sum_noalloc(fx_ctx* ctx, const void* fi, const uint8_t* flags, u
 	return mass_sum_with(ctx, fi, flags, t, ctx->scratch, ctx->scratch + NOALLOC_MASS_PARTIALS, out);
 }
 
-static uint64_t ddf_bytes(const fx_ctx* ctx) {
-	return ctx->N * (uint64_t)ctx->cfg.velocity_set * (ctx->cfg.storage == FX_FP32 ? 4u : 2u);
-}
 static int adjoint_layout(const fx_ctx* ctx, const fx_adjoint_config* cfg, uint64_t& k, uint64_t& checkpoints, uint64_t& bytes) {
 	if(!ctx || !cfg) return fail(FX_ERR_ARG, "null argument");
 	if(ctx->cfg.extensions & (FX_MOVING_BOUNDARIES | FX_SUBGRID))
@@ -763,18 +874,18 @@ int fx_adjoint_create(fx_ctx* ctx, const fx_adjoint_config* cfg, fx_adjoint** ou
 	int rc = adjoint_layout(ctx, cfg, k, checkpoints, bytes);
 	if(rc != FX_OK) return rc;
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	size_t free_b = 0, total_b = 0;
-	FX_HIP(hipMemGetInfo(&free_b, &total_b));
-	if(bytes > (uint64_t)free_b) return fail(FX_ERR_MEMORY, "adjoint workspace of " + std::to_string(bytes) + " bytes does not fit the free device memory");
+	uint64_t free_b = 0;
+	FX_HIP(free_memory(ctx->device, bytes, &free_b));
+	if(bytes > free_b) return fail(FX_ERR_MEMORY, "adjoint workspace of " + std::to_string(bytes) + " bytes does not fit the free device memory");
 	fx_adjoint* adj = new fx_adjoint();
 	adj->ctx = ctx; adj->cfg = *cfg; adj->k = k; adj->checkpoints = checkpoints; adj->fi_bytes = ddf_bytes(ctx);
 	adj->obj_blocks = ((uint64_t)ctx->cfg.Ny * ctx->cfg.Nz + 255u) / 256u;
-	hipError_t e = hipMalloc(&adj->ckpt, checkpoints * adj->fi_bytes);
-	if(e == hipSuccess) e = hipMalloc(&adj->work_fi, adj->fi_bytes);
-	if(e == hipSuccess) e = hipMalloc(&adj->moments, k * 4u * ctx->N * sizeof(float));
-	if(e == hipSuccess) e = hipMalloc(&adj->lambda, (uint64_t)ctx->cfg.velocity_set * ctx->N * sizeof(float));
-	if(e == hipSuccess) e = hipMalloc(&adj->partial, adj->obj_blocks * sizeof(double));
-	if(e == hipSuccess) e = hipMalloc(&adj->acc, sizeof(double));
+	hipError_t e = allocate_device(ctx->device, (void**)&adj->ckpt, checkpoints * adj->fi_bytes);
+	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->work_fi, adj->fi_bytes);
+	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->moments, k * 4u * ctx->N * sizeof(float));
+	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->lambda, (uint64_t)ctx->cfg.velocity_set * ctx->N * sizeof(float));
+	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->partial, adj->obj_blocks * sizeof(double));
+	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->acc, sizeof(double));
 	if(e != hipSuccess) { fx_adjoint_destroy(adj); return fail(FX_ERR_MEMORY, std::string("adjoint workspace: ") + hipGetErrorString(e)); }
 	*out = adj;
 	return FX_OK;
@@ -861,15 +972,17 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 	const fx_adjoint_config& c = adj->cfg;
 	FX_HIP(hipMemsetAsync(adj->acc, 0, sizeof(double), ctx->stream));
 	FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-	fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, 0u, fx_, fy_, fz_, F, alpha);
-	for(uint64_t t = 0; t < c.steps; t++) {
+	const fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, 0u, fx_, fy_, fz_, F, alpha);
+	for(uint64_t t = 0, n = 0; t < c.steps; t += n) {
 		if(t % adj->k == 0u) FX_HIP(hipMemcpyAsync(adj->ckpt + (t / adj->k) * adj->fi_bytes, fi, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
 		if(t >= c.window_begin) {
 			rc = objective_accumulate(ctx, fi, flags, t, c.plane_x, adj->partial, adj->obj_blocks, adj->acc);
 			if(rc != FX_OK) return rc;
+			n = 1u; // the objective looks at every step
+		} else {
+			n = std::min(adj->k - t % adj->k, c.window_begin - t); // up to the next checkpoint or the window (window_begin < steps)
 		}
-		a.odd = (uint32_t)(t & 1u);
-		ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+		queue_steps(ctx, a, t, n);
 	}
 	rc = check_launch("forward");
 	if(rc != FX_OK) return rc;

@@ -2,6 +2,7 @@
 // storage, collision); filled by the per-velocity-set translation units.
 #pragma once
 #include "lbm_device.hpp"
+#include "lbm_two_steps.hpp"
 
 namespace fx {
 
@@ -96,12 +97,50 @@ inline size_t occupancy_lds(uint32_t waves_per_simd, uint32_t block_threads, siz
 	return lds;
 }
 
+// Launch of k_two_steps: a block per tile of width x height columns and segment of zlen
+// planes; tiles of at most 128 x 5 columns, 64 x 13 on rows of at most 64 cells.
+struct TwoStepShape {
+	bool wide = false;
+	uint32_t width = 0, height = 0, zlen = 0, tiles_x = 0, tiles_y = 0, tiles = 0, grid = 0; // grid 0: not used
+};
+constexpr uint32_t TWO_STEP_WIDE_X = 128u, TWO_STEP_WIDE_Y = 5u, TWO_STEP_NARROW_X = 64u, TWO_STEP_NARROW_Y = 13u;
+// One block runs per CU (registers).  A plane takes a time of about height + 3 units (loads and
+// collisions per row, barriers), a block as many planes as its segment, two beside it and
+// about two planes' time to start, and the blocks run in rounds of one per CU: the shape is
+// the one with the least rounds * (zlen + 4) * (height + 3) among heights of 4 and more (2 and
+// 3 rows measured 5 to 25 % slower at 64^3 to 256^3: the two border rows are loaded and
+// collided twice).  Measured best heights, 128 wide: 4 at 96^3, 128^3, 256^3, 5 at 160^3 and
+// 200^3; 64 wide: 4 at 32^3 and 64^3, 8 at 64x256x256.
+inline TwoStepShape two_step_shape(uint32_t Nx, uint32_t Ny, uint32_t Nz, uint32_t cus) {
+	TwoStepShape s;
+	s.wide = Nx > TWO_STEP_NARROW_X;
+	const uint32_t TX = s.wide ? TWO_STEP_WIDE_X : TWO_STEP_NARROW_X, TY = s.wide ? TWO_STEP_WIDE_Y : TWO_STEP_NARROW_Y;
+	const uint32_t nx = (Nx + TX - 1u) / TX;
+	s.width = ((Nx + nx - 1u) / nx + 31u) / 32u * 32u; // whole 128-byte lines, <= TX
+	s.tiles_x = (Nx + s.width - 1u) / s.width;
+	const uint64_t capacity = cus ? cus : 1u;
+	uint64_t best = ~0ull;
+	for(uint32_t h = 4u; h <= TY; h++) {
+		const uint32_t tiles_y = (Ny + h - 1u) / h;
+		const uint64_t columns = (uint64_t)s.tiles_x * tiles_y;
+		for(uint32_t n = 1u; n <= Nz; n++) { // segments
+			const uint32_t zlen = (Nz + n - 1u) / n;
+			const uint64_t blocks = columns * ((Nz + zlen - 1u) / zlen);
+			if(n > 1u && blocks > 4u * capacity) break; // shorter segments only add planes
+			const uint64_t cost = (blocks + capacity - 1u) / capacity * (zlen + 4u) * (h + 3u);
+			if(cost < best) { best = cost; s.height = h; s.zlen = zlen; s.tiles_y = tiles_y; s.tiles = (uint32_t)blocks; }
+		}
+	}
+	s.grid = (s.tiles + 7u) / 8u * 8u;
+	return s;
+}
 // Grid of the adjoint kernels (record pass and adjoint step): XCD-mapped, full occupancy.
 inline LaunchShape adjoint_shape(uint32_t Nx, uint32_t Ny, uint32_t Nz) { return stream_shape(Nx, Ny, Nz, true); }
 
 typedef void (*lattice_fn)(const LbmArgs&, const LaunchShape&, hipStream_t);
 typedef void (*mass_fn)(const LbmArgs&, const LaunchShape&, hipStream_t, double*);
 typedef void (*record_fn)(const LbmArgs&, const LaunchShape&, hipStream_t, float*);
+typedef void (*two_steps_fn)(const LbmArgs&, void*, const TwoStepShape&, hipStream_t);
 typedef void (*adjoint_fn)(const AdjointArgs&, const LaunchShape&, hipStream_t);
 typedef void (*objective_fn)(const LbmArgs&, uint32_t, hipStream_t, double*);
 typedef void (*transfer_fn)(void* fi, void* buffer_p, void* buffer_m, uint32_t Nx, uint32_t Ny, uint32_t Nz, uint32_t axis, bool insert,
@@ -127,6 +166,7 @@ struct LbmKernels {
 	bool stream_collide_buffer;       // buffer instructions on the row grid (DDFs below 4 GiB)
 	bool stream_collide_pair_buffer;  // the same for k_stream_collide_pair
 	bool stream_collide_linear_buffer; // the same on the cell-linear grid
+	two_steps_fn two_steps;           // two time steps in one launch (k_two_steps), null where it does not pay
 };
 
 constexpr uint32_t EXT_ALL = EXT_VOLUME_FORCE | EXT_FORCE_FIELD | EXT_EQUILIBRIUM_BOUNDARIES | EXT_UPDATE_FIELDS | EXT_POROSITY |
@@ -261,6 +301,31 @@ inline bool use_linear_grid(const LbmKernels& k, uint32_t Nx, uint32_t elem_byte
 	return !rows_on_lines(Nx, elem_bytes) || (k.stream_collide_linear_large && N * q * elem_bytes > LARGE_DDF_BYTES);
 }
 
+// Two steps per launch (k_two_steps) against single steps, fx_lbm_run, MI355X, microseconds
+// per step.  FP32 only: the 16-bit kernels are bound by instructions, not bytes (D3Q19 FP16S
+// 256^3: 240 to 260 against 207).  D3Q19 SRT: 64^3 9.4 -> 7.6, 128^3 57.7 -> 38.3, 256^3 399
+// -> 267, 512x256x256 894 -> 560, 512^3 3723 -> 2200, 1000x250x250 1818 -> 1195, 300^3 783
+// -> 635; TRT VOLUME_FORCE 256^3 444 -> 344; porous TRT 256^3 461 -> 397; D3Q27 TRT
+// EQUILIBRIUM_BOUNDARIES 256^3 663 -> 459.  The all-extension kernels lost up to 2x (D3Q27
+// TRT spills) and gained at most 7 % (D3Q19 SRT): not taken.
+constexpr bool tune_two_steps(int Q, uint32_t ST, bool TRT, uint32_t EXT) { return ST == ST_FP32 && EXT != EXT_ALL; }
+// Lattices that gain.  The step t of a tile's border cells is taken twice and lanes beyond a
+// row's end idle, which costs the more the more arithmetic a cell has (weight: one each for
+// VOLUME_FORCE, POROSITY, TRT and D3Q27), and a launch takes longer to start.
+// Lanes in use, Nx over the tiles' width: weight 0 to 2 gained 2 to 42 % at 55 to 63 % (140^3,
+// 72x128x128, 160^3) and -4 to +2 % at 51 % (130^3, 65^3); rows of at most 64 cells +1 % at
+// 38 % (Nx = 24), -16 % at 25 %; weight 3 and 4 -12 to +2 % at 56 to 78 % (160^3, 200^3), +6 to
+// +27 % above 90 %.  Cells: weight 0 -3 % at 32^3, +6 % at 40^3, +20 % at 48^3; weight 1 +10 to
+// +15 % at 64^3, weight 2 -2 to +4 % there and +3 to +22 % at 128x64x64, weight 3 and 4 -11 to
+// -3 % and +1 to +6 %.  One or two planes: 400x400x1 -20 %, x2 -5 %, x3 +1 %, x4 +4 %; rows of
+// one plane: 400x1x400 -20 %, 1000x1x300 -3 %, 1000x2x300 +37 %.
+inline bool two_steps_pay(const TwoStepShape& s, uint32_t Nx, uint32_t Ny, uint32_t Nz, uint32_t q, bool trt, uint32_t ext) {
+	const uint32_t weight = ((ext & (EXT_VOLUME_FORCE | EXT_POROSITY)) ? 1u : 0u) + ((ext & EXT_POROSITY) ? 1u : 0u) + (trt ? 1u : 0u) + (q == 27u ? 1u : 0u);
+	if(Ny < 2u || Nz < 4u || (uint64_t)Nx * Ny * Nz <= 65536ull << weight) return false;
+	const uint64_t lanes = (uint64_t)s.tiles_x * (s.wide ? TWO_STEP_WIDE_X : TWO_STEP_NARROW_X), percent = Nx * 100ull / lanes;
+	return percent >= (weight > 2u ? 90u : s.wide ? 55u : 40u);
+}
+
 // Kernel set of one (velocity set, storage, collision) variant; EXT = 0 instantiates the
 // extension-free kernels, EXT_ALL the ones that read the runtime extension mask.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
@@ -319,6 +384,13 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		const uint64_t cells = (uint64_t)a.Ny * a.Nz;
 		k_objective_partial<Q, ST><<<(unsigned)((cells + 255u) / 256u), 256, 0, st>>>(a, plane_x, p);
 	}
+	static void two_steps(const LbmArgs& a, void* dst, const TwoStepShape& s, hipStream_t st) {
+		if constexpr(two_step) {
+			const TwoStepArgs g = {a, dst, s.tiles_x, s.tiles_y, s.tiles, s.width, s.height, s.zlen};
+			if(s.wide) k_two_steps<Q, TRT, EXT, TWO_STEP_WIDE_X, TWO_STEP_WIDE_Y><<<s.grid, two_step_threads(TWO_STEP_WIDE_X, s.height), 0, st>>>(g);
+			else k_two_steps<Q, TRT, EXT, TWO_STEP_NARROW_X, TWO_STEP_NARROW_Y><<<s.grid, two_step_threads(TWO_STEP_NARROW_X, s.height), 0, st>>>(g);
+		}
+	}
 	// Launch tuning of stream_collide: residency cap in waves per SIMD (0 = none) and grid.
 	static constexpr uint32_t waves_cap = tune_waves_cap(Q, ST, EXT);
 	static constexpr bool xcd_map = tune_xcd_map(Q, ST, EXT);
@@ -328,6 +400,7 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 	static constexpr bool buffer = tune_buffer(Q, ST, TRT, EXT);
 	static constexpr bool pair_buffer = tune_pair_buffer(Q, ST, TRT, EXT);
 	static constexpr bool linear_buffer = tune_linear_buffer(Q, ST, TRT, EXT);
+	static constexpr bool two_step = tune_two_steps(Q, ST, TRT, EXT);
 	template<int AXIS> static void transfer_axis(void* fi, void* bp, void* bm, uint32_t Nx, uint32_t Ny, uint32_t Nz, bool insert, uint32_t odd, hipStream_t st) {
 		typedef typename Storage<ST>::E E;
 		const uint64_t A = AXIS == 0 ? (uint64_t)Ny * Nz : AXIS == 1 ? (uint64_t)Nx * Nz : (uint64_t)Nx * Ny;
@@ -344,7 +417,7 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		static const LbmKernels k = {initialize, stream_collide, update_fields, update_force_field, mass_partial, waves_cap,
 		                             stream_collide_record, adjoint_step, objective_partial, xcd_map, transfer_fi,
 		                             update_moving_boundaries, tune_linear_large(Q, ST, EXT), linear_xcd, pairs, offsets32, buffer, pair_buffer,
-	                             linear_buffer};
+	                             linear_buffer, two_step ? two_steps : nullptr};
 		return &k;
 	}
 };

@@ -176,12 +176,17 @@ class LBM:
         sync_each_step=True reproduces the reference's per-step finish_queue (src/lbm.cpp:951)."""
         if not self.initialized:
             self.initialize()
-        for _ in range(int(steps)):
-            check(self.ctx.lib.fx_lbm_stream_collide(*self._step_args(), self.t, self.fx, self.fy, self.fz,
-                                                     self._ptr(self.F), self._ptr(self.porosity)))
-            if sync_each_step:
+        steps = int(steps)
+        if sync_each_step:
+            for _ in range(steps):
+                check(self.ctx.lib.fx_lbm_stream_collide(*self._step_args(), self.t, self.fx, self.fy, self.fz,
+                                                         self._ptr(self.F), self._ptr(self.porosity)))
                 self.ctx.sync()
-            self.t += 1
+                self.t += 1
+        elif steps > 0:
+            check(self.ctx.lib.fx_lbm_run(*self._step_args(), self.t, steps, self.fx, self.fy, self.fz, self._ptr(self.F),
+                                          self._ptr(self.porosity), None))
+            self.t += steps
         if self.extensions & _abi.FX_UPDATE_FIELDS:
             self.t_last_update_fields = self.t
         self.ctx.sync()
