@@ -1175,19 +1175,31 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_record(LbmArgs a, floa
 	stream_collide_cell<Q, ST, TRT, EXT & ~(EXT_MOVING_BOUNDARIES | EXT_SUBGRID), true, XCD, LIN>(a, moments);
 }
 
-// update_fields (src/kernel.cpp:1794-1870)
-template<int Q, uint32_t ST, uint32_t EXT>
+// update_fields (src/kernel.cpp:1794-1870), on the grids of stream_collide (cell_coords).
+// Bound by memory: each DDF read once, 16 bytes of fields written per cell.  The fields are
+// streamed with non-temporal stores from UPDATE_FIELDS_STREAM cells on: D3Q19 256^3 FP32 283 ->
+// 250 us (6.2 TB/s), 128^3 35.5 -> 32.3, 96^3 FP16S 11.0 -> 10.9, 128x64x64 equal, 64^3 FP16S
+// 4.7 -> 5.2.  Rows off the cache lines on the cell-linear grid instead of the row grid:
+// 200^3 FP32 160 -> 106 us, FP16C 87 -> 70, 160x120x100 FP16S 25.7 -> 20.5, 201x75x99 FP32 31.8
+// -> 25.0.  BUF on the row grid: rows of several blocks, 384x192x192 FP16S 130 -> 121 and
+// D3Q27 FP16C 169 -> 155 (rows of one block: 256^3 D3Q19 -3 %, D3Q27 +7 %, 128^3 +5 to +11 %).
+constexpr uint64_t UPDATE_FIELDS_STREAM = 1ull << 19;
+template<int Q, uint32_t ST, uint32_t EXT, bool XCD, bool LIN, bool BUF>
 __global__ __launch_bounds__(BLOCK) void k_update_fields(LbmArgs a) {
 	a.ext &= EXT;
-	const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x;
-	if(x >= a.Nx) return;
-	const Site s = make_site(x, blockIdx.y, blockIdx.z, a.Nx, a.Ny, a.Nz);
+	uint32_t x, y, z;
+	if(!cell_coords<XCD, LIN>(a, x, y, z)) return;
+	const Site s = make_site(x, y, z, a.Nx, a.Ny, a.Nz);
 	const uint64_t n = s.n();
 	const uint32_t flagsn = a.flags[n];
 	const uint32_t bo = flagsn & TYPE_BO;
 	if(bo == TYPE_S || (flagsn & TYPE_SU) == TYPE_G) return;
 	float fhn[Q];
-	load_f<Q, ST>((const typename Storage<ST>::E*)a.fi, a.N, s, a.odd, fhn);
+	typename Storage<ST>::E r[Q];
+	load_raw<Q, ST, false, LIN, false, BUF>((const typename Storage<ST>::E*)a.fi, a.N, s, a.odd, r);
+	if constexpr(ST == ST_FP16S) __builtin_amdgcn_sched_barrier(0); // every load before the first conversion
+#pragma unroll
+	for(int i = 0; i < Q; i++) fhn[i] = Storage<ST>::decode(r[i]);
 	if((a.ext & EXT_MOVING_BOUNDARIES) && bo == TYPE_MS) moving_boundaries<Q>(a, s, fhn);
 	float rhon, uxn, uyn, uzn;
 	calc_rho_u<Q>(fhn, rhon, uxn, uyn, uzn);
@@ -1196,10 +1208,34 @@ __global__ __launch_bounds__(BLOCK) void k_update_fields(LbmArgs a) {
 	const float alphan = (a.ext & EXT_POROSITY) ? a.alpha[n] : 0.0f;
 	force_block(a.ext, rhon, uxn, uyn, uzn, fxn, fyn, fzn, alphan);
 	if(!((a.ext & EXT_EQUILIBRIUM_BOUNDARIES) && bo == TYPE_E)) {
-		a.rho[n] = rhon; a.u[n] = uxn; a.u[a.N + n] = uyn; a.u[2ull * a.N + n] = uzn;
+		if(a.N >= UPDATE_FIELDS_STREAM) {
+			__builtin_nontemporal_store(rhon, a.rho + n);
+			__builtin_nontemporal_store(uxn, a.u + n); __builtin_nontemporal_store(uyn, a.u + a.N + n); __builtin_nontemporal_store(uzn, a.u + 2ull * a.N + n);
+		} else {
+			a.rho[n] = rhon; a.u[n] = uxn; a.u[a.N + n] = uyn; a.u[2ull * a.N + n] = uzn;
+		}
 	}
 }
 
+// f(n) for the cells n of [c0, c0 + 256) whose flags & mask equal value, each on one lane of a
+// wave (all 64 lanes call it): every lane reads four flags at once, and the runs of 64 cells
+// that hold a match are then taken one cell per lane, so what f reads is consecutive.
+constexpr uint32_t SCAN_CELLS = 256u;
+template<class F> __device__ __forceinline__ void scan_flags(const uint8_t* flags, uint64_t N, uint64_t c0, uint32_t mask, uint32_t value, F&& f) {
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint64_t mine = c0 + lane * 4u;
+	uint32_t word = (value ^ 0xFFu) * 0x01010101u; // matches nothing
+	if(mine + 4u <= N && ((uint64_t)flags & 3u) == 0u) word = *(const uint32_t*)(flags + mine);
+	else for(uint32_t j = 0; j < 4u; j++) if(mine + j < N) word = (word & ~(0xFFu << (8u * j))) | ((uint32_t)flags[mine + j] << (8u * j));
+	const uint32_t t = (word & (mask * 0x01010101u)) ^ (value * 0x01010101u); // a zero byte: a match
+	uint64_t lanes = __ballot(((t - 0x01010101u) & ~t & 0x80808080u) != 0u); // lanes 16r .. 16r+15: run r
+	while(lanes) {
+		const uint32_t run = (uint32_t)__builtin_ctzll(lanes) >> 4;
+		lanes &= ~(0xFFFFull << (run * 16u));
+		const uint32_t w = (uint32_t)__shfl((int)t, (int)(run * 16u + (lane >> 2)));
+		if(((w >> (8u * (lane & 3u))) & 0xFFu) == 0u) f(c0 + run * 64u + lane);
+	}
+}
 // update_force_field (src/kernel.cpp:1873-1884): momentum exchange on solid cells
 template<int Q, uint32_t ST>
 __global__ __launch_bounds__(BLOCK) void k_update_force_field(LbmArgs a) {

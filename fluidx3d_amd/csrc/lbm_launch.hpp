@@ -360,7 +360,21 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		}
 		k_stream_collide<Q, ST, TRT, EXT, xcd_map, false><<<s.grid, s.block, s.lds, st>>>(b);
 	}
-	static void update_fields(const LbmArgs& a, const LaunchShape& s, hipStream_t st) { k_update_fields<Q, ST, (EXT == 0u ? 0u : EXT_ALL)><<<s.grid, s.block, 0, st>>>(a); }
+	static void update_fields(const LbmArgs& a, const LaunchShape& s, hipStream_t st) {
+		LbmArgs b = a;
+		b.xchunks = s.xchunks;
+		if(s.lin) {
+			if constexpr(linear_buffer) {
+				if(s.buf) { k_update_fields<Q, ST, EXT, linear_xcd, true, true><<<s.grid, s.block, 0, st>>>(b); return; }
+			}
+			k_update_fields<Q, ST, EXT, linear_xcd, true, false><<<s.grid, s.block, 0, st>>>(b);
+		} else if(s.xchunks > 0u) {
+			if constexpr(ST != ST_FP32) {
+				if(s.buf) { k_update_fields<Q, ST, EXT, true, false, true><<<s.grid, s.block, 0, st>>>(b); return; }
+			}
+			k_update_fields<Q, ST, EXT, true, false, false><<<s.grid, s.block, 0, st>>>(b);
+		} else k_update_fields<Q, ST, EXT, false, false, false><<<s.grid, s.block, 0, st>>>(b);
+	}
 	static void update_force_field(const LbmArgs& a, const LaunchShape& s, hipStream_t st) { k_update_force_field<Q, ST><<<s.grid, s.block, 0, st>>>(a); }
 	static void mass_partial(const LbmArgs& a, const LaunchShape& s, hipStream_t st, double* p) { k_mass_partial<Q, ST><<<s.grid, s.block, 0, st>>>(a, p); }
 	static void update_moving_boundaries(const LbmArgs& a, const LaunchShape& s, hipStream_t st) { k_update_moving_boundaries<Q><<<s.grid, s.block, 0, st>>>(a); }

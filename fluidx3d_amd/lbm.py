@@ -217,24 +217,27 @@ class LBM:
         self.fx, self.fy, self.fz = float(fx), float(fy), float(fz)
 
     # -- forces (FORCE_FIELD) ---------------------------------------------------------
-    def update_force_field(self):
+    def _update_force_field_if_stale(self):
         if self.F is None:
             raise ValueError("FORCE_FIELD is not enabled")
         if self.t_last_force_field != self.t:
             check(self.ctx.lib.fx_lbm_update_force_field(self.ctx.h, self.fi, self.flags.device, self.t, self.F.device))
             self.t_last_force_field = self.t
+
+    def update_force_field(self):
+        self._update_force_field_if_stale()
         self.ctx.sync()
 
     def object_force(self, flag_marker=TYPE_S):
         import ctypes
-        self.update_force_field()
+        self._update_force_field_if_stale()
         out = (ctypes.c_double * 3)()
         check(self.ctx.lib.fx_lbm_object_force(self.ctx.h, self.F.device, self.flags.device, flag_marker, out))
         return np.array(out[:])
 
     def object_torque(self, rotation_center, flag_marker=TYPE_S):
         import ctypes
-        self.update_force_field()
+        self._update_force_field_if_stale()
         out = (ctypes.c_double * 3)()
         c = [float(v) for v in rotation_center]
         check(self.ctx.lib.fx_lbm_object_torque(self.ctx.h, self.F.device, self.flags.device, flag_marker, c[0], c[1], c[2], out))
