@@ -171,11 +171,19 @@ struct LbmKernels {
 
 constexpr uint32_t EXT_ALL = EXT_VOLUME_FORCE | EXT_FORCE_FIELD | EXT_EQUILIBRIUM_BOUNDARIES | EXT_UPDATE_FIELDS | EXT_POROSITY |
                              EXT_PRECISE_DENSITY | EXT_MOVING_BOUNDARIES | EXT_SUBGRID;
+// Unforced flows with the subgrid model, and with moving walls too: what aerodynamics and
+// cavity scenes switch on.  Against the all-extension kernel (run with the same extensions):
+// D3Q19 SRT SUBGRID 256^3 FP16S 254 -> 239 us, FP16C 257 -> 233, D3Q27 TRT FP16C 432 -> 338;
+// MOVING_BOUNDARIES + SUBGRID 128^3 D3Q19 SRT FP16S 39.2 -> 34.4; EQUILIBRIUM_BOUNDARIES +
+// FORCE_FIELD + MOVING_BOUNDARIES 256^3 D3Q19 FP16S 289 -> 247 (SRT), 305 -> 251 (TRT); FP32
+// single steps -1 to +12 %.
+constexpr uint32_t EXT_LES = EXT_EQUILIBRIUM_BOUNDARIES | EXT_FORCE_FIELD | EXT_SUBGRID;
+constexpr uint32_t EXT_LES_MOVING = EXT_LES | EXT_MOVING_BOUNDARIES;
 
 // Measured launch tuning (see KernelSet), MI355X, 256^3 to 1536x768x768:
 // - FP32 kernels (non-temporal DDF access) stream fastest with fewer concurrent DDF
 //   streams: plain D3Q19/D3Q27 at 3 waves/SIMD (+11 % / +3 % over full occupancy),
-//   D3Q19 with EQUILIBRIUM_BOUNDARIES (+FORCE_FIELD) at 4 (+2-4 %), D3Q19 with
+//   D3Q19 with EQUILIBRIUM_BOUNDARIES (+FORCE_FIELD; and SUBGRID, MOVING_BOUNDARIES) at 4 (+2-4 %), D3Q19 with
 //   VOLUME_FORCE (+POROSITY) at 3 (+4 %); the generic all-extension kernel is not capped;
 // - the 2-byte formats (non-temporal too) need full occupancy;
 // - on rows of several blocks the XCD-mapped grid gains 9-24 % for FP16S, 6-10 % for FP32
@@ -189,7 +197,7 @@ constexpr uint32_t tune_waves_cap(int Q, uint32_t ST, uint32_t EXT) {
 	if(ST != ST_FP32) return 0u;
 	if(EXT == 0u) return 3u;
 	if(Q != 19) return 0u;
-	if(EXT == EXT_EQUILIBRIUM_BOUNDARIES || EXT == (EXT_EQUILIBRIUM_BOUNDARIES | EXT_FORCE_FIELD)) return 4u;
+	if(EXT == EXT_EQUILIBRIUM_BOUNDARIES || EXT == (EXT_EQUILIBRIUM_BOUNDARIES | EXT_FORCE_FIELD) || EXT == EXT_LES || EXT == EXT_LES_MOVING) return 4u;
 	if(EXT == EXT_VOLUME_FORCE || EXT == (EXT_VOLUME_FORCE | EXT_POROSITY | EXT_PRECISE_DENSITY)) return 3u;
 	return 0u;
 }
@@ -306,12 +314,13 @@ inline bool use_linear_grid(const LbmKernels& k, uint32_t Nx, uint32_t elem_byte
 // 256^3: 240 to 260 against 207).  D3Q19 SRT: 64^3 9.4 -> 7.6, 128^3 57.7 -> 38.3, 256^3 399
 // -> 267, 512x256x256 894 -> 560, 512^3 3723 -> 2200, 1000x250x250 1818 -> 1195, 300^3 783
 // -> 635; TRT VOLUME_FORCE 256^3 444 -> 344; porous TRT 256^3 461 -> 397; D3Q27 TRT
-// EQUILIBRIUM_BOUNDARIES 256^3 663 -> 459.  The all-extension kernels lost up to 2x (D3Q27
-// TRT spills) and gained at most 7 % (D3Q19 SRT): not taken.
+// EQUILIBRIUM_BOUNDARIES 256^3 663 -> 459.  SUBGRID D3Q19 SRT
+// 256^3 420 -> 313, MOVING_BOUNDARIES 421 -> 272.  The all-extension kernels lost up to 2x
+// (D3Q27 TRT spills) and gained at most 7 % (D3Q19 SRT): not taken.
 constexpr bool tune_two_steps(int Q, uint32_t ST, bool TRT, uint32_t EXT) { return ST == ST_FP32 && EXT != EXT_ALL; }
 // Lattices that gain.  The step t of a tile's border cells is taken twice and lanes beyond a
 // row's end idle, which costs the more the more arithmetic a cell has (weight: one each for
-// VOLUME_FORCE, POROSITY, TRT and D3Q27), and a launch takes longer to start.
+// VOLUME_FORCE, POROSITY, TRT and D3Q27, two for SUBGRID), and a launch takes longer to start.
 // Lanes in use, Nx over the tiles' width: weight 0 to 2 gained 2 to 42 % at 55 to 63 % (140^3,
 // 72x128x128, 160^3) and -4 to +2 % at 51 % (130^3, 65^3); rows of at most 64 cells +1 % at
 // 38 % (Nx = 24), -16 % at 25 %; weight 3 and 4 -12 to +2 % at 56 to 78 % (160^3, 200^3), +6 to
@@ -320,7 +329,7 @@ constexpr bool tune_two_steps(int Q, uint32_t ST, bool TRT, uint32_t EXT) { retu
 // -3 % and +1 to +6 %.  One or two planes: 400x400x1 -20 %, x2 -5 %, x3 +1 %, x4 +4 %; rows of
 // one plane: 400x1x400 -20 %, 1000x1x300 -3 %, 1000x2x300 +37 %.
 inline bool two_steps_pay(const TwoStepShape& s, uint32_t Nx, uint32_t Ny, uint32_t Nz, uint32_t q, bool trt, uint32_t ext) {
-	const uint32_t weight = ((ext & (EXT_VOLUME_FORCE | EXT_POROSITY)) ? 1u : 0u) + ((ext & EXT_POROSITY) ? 1u : 0u) + (trt ? 1u : 0u) + (q == 27u ? 1u : 0u);
+	const uint32_t weight = ((ext & (EXT_VOLUME_FORCE | EXT_POROSITY)) ? 1u : 0u) + ((ext & EXT_POROSITY) ? 1u : 0u) + ((ext & EXT_SUBGRID) ? 2u : 0u) + (trt ? 1u : 0u) + (q == 27u ? 1u : 0u);
 	if(Ny < 2u || Nz < 4u || (uint64_t)Nx * Ny * Nz <= 65536ull << weight) return false;
 	const uint64_t lanes = (uint64_t)s.tiles_x * (s.wide ? TWO_STEP_WIDE_X : TWO_STEP_NARROW_X), percent = Nx * 100ull / lanes;
 	return percent >= (weight > 2u ? 90u : s.wide ? 55u : 40u);
@@ -451,6 +460,8 @@ template<int Q, uint32_t ST> const LbmKernels* kernels_for(bool trt, uint32_t ex
 	if((ext & ~VF) == 0u) return pick<Q, ST, VF>(trt);
 	if((ext & ~(E | FF)) == 0u) return pick<Q, ST, E | FF>(trt);
 	if((ext & ~POROUS) == 0u) return pick<Q, ST, POROUS>(trt);
+	if((ext & ~EXT_LES) == 0u) return pick<Q, ST, EXT_LES>(trt);
+	if((ext & ~EXT_LES_MOVING) == 0u) return pick<Q, ST, EXT_LES_MOVING>(trt);
 	return pick<Q, ST, EXT_ALL>(trt);
 }
 // One translation unit per (velocity set, storage) instantiates each table.

@@ -79,7 +79,7 @@ __global__ __launch_bounds__((two_step_threads(TX, TY))) void k_two_steps(TwoSte
 	// consecutive blocks go to the 8 XCDs in turn: each XCD takes a run of neighbouring tiles
 	const uint32_t per = gridDim.x >> 3, tile = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
 	if(tile >= g.tiles) return;
-	static_assert(!(EXT & (EXT_UPDATE_FIELDS | EXT_MOVING_BOUNDARIES)), "rho and u are not written, neighbours' flags not read");
+	static_assert(!(EXT & EXT_UPDATE_FIELDS), "step t of a border cell would write rho and u beside the block that owns it");
 	LbmArgs a = g.a;
 	a.ext &= EXT;
 	const uint32_t Nx = a.Nx, Ny = a.Ny, Nz = a.Nz;
@@ -146,6 +146,7 @@ __global__ __launch_bounds__((two_step_threads(TX, TY))) void k_two_steps(TwoSte
 		} else {
 			float f[Q];
 			static_for<0, Q, 1>([&](auto c) __attribute__((always_inline)) { constexpr int i = decltype(c)::value; f[i] = in[i]; });
+			if((a.ext & EXT_MOVING_BOUNDARIES) && (flagsn & TYPE_BO) == TYPE_MS) moving_boundaries<Q>(a, make_site(x, y, z, Nx, Ny, Nz), f);
 			collide_cell<Q, TRT, EXT, false, false, shared_pair_difference(Q, EXT, false)>(a, z * P + col, flagsn & TYPE_BO, f, nullptr);
 			static_for<0, Q, 1>([&](auto c) __attribute__((always_inline)) { constexpr int i = decltype(c)::value; out[i] = f[i]; });
 		}

@@ -102,6 +102,11 @@ CASES = [
     ((125, 91, 25), 19, "SRT", POROUS),
     ((123, 91, 53), 19, "TRT", POROUS),
     ((254, 71, 61), 27, "TRT", POROUS),
+    ((160, 70, 33), 19, "SRT", ("SUBGRID",)),
+    ((128, 70, 61), 19, "TRT", ("EQUILIBRIUM_BOUNDARIES", "SUBGRID")),
+    ((150, 40, 33), 19, "SRT", ("MOVING_BOUNDARIES",)),
+    ((100, 63, 47), 27, "SRT", ("MOVING_BOUNDARIES", "FORCE_FIELD", "EQUILIBRIUM_BOUNDARIES")),
+    ((128, 91, 97), 27, "TRT", ("MOVING_BOUNDARIES", "SUBGRID")),
 ]
 
 
