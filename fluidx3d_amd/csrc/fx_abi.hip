@@ -588,7 +588,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 		ctx->shape_sc = fx::linear_shape(N, ctx->k->stream_collide_linear_xcd);
 		ctx->shape_sc.buf = ctx->k->stream_collide_linear_buffer && N * cfg->velocity_set * eb <= 0xFFFFFFFFull;
 		ctx->shape_adj = fx::linear_shape(N, false);
-	} else if(ctx->k->stream_collide_pairs && fx::pair_rows(cfg->Nx)) {
+	} else if(ctx->k->stream_collide_pairs && fx::pair_rows(cfg->Nx) && fx::pair_extensions(cfg->storage, cfg->collision == FX_TRT, cfg->extensions)) {
 		ctx->shape_sc = fx::pair_shape(cfg->Nx, cfg->Ny, cfg->Nz);
 		ctx->shape_sc.buf = ctx->k->stream_collide_pair_buffer && N * cfg->velocity_set * eb <= 0xFFFFFFFFull;
 	} else if(ctx->k->stream_collide_buffer && N * cfg->velocity_set * eb <= 0xFFFFFFFFull) {

@@ -1045,7 +1045,7 @@ __device__ __forceinline__ gword* word_at(gcode* p, uint32_t x) { return (gword*
 // no 64-bit store addresses rebuilt in vector registers after the collision.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool BUF = false>
 __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
-	static_assert(ST != ST_FP32 && !(EXT & EXT_MOVING_BOUNDARIES), "16-bit codes only; populations as decoded");
+	static_assert(ST != ST_FP32, "16-bit codes only");
 	a.ext &= EXT;
 	typedef Storage<ST> S;
 	uint32_t chunk, y, z;
@@ -1120,6 +1120,7 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 			if constexpr(ST == ST_FP16C) f[i] = S::decode_low(P[i]);
 			else f[i] = S::decode((uint16_t)P[i]);
 		}
+		if((a.ext & EXT_MOVING_BOUNDARIES) && (flA & TYPE_BO) == TYPE_MS) moving_boundaries<Q>(a, s, f);
 		collide_cell<Q, TRT, EXT, false, shared_division(ST, EXT), shared_pair_difference(Q, EXT, BUF)>(a, n, flA & TYPE_BO, f, nullptr);
 #pragma unroll
 		for(int i = 0; i < Q; i++) P[i] = (P[i] & 0xFFFF0000u) | S::encode_word(f[i]);
@@ -1131,6 +1132,7 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 	if(liveB) {
 #pragma unroll
 		for(int i = 0; i < Q; i++) f[i] = S::decode((uint16_t)(P[i] >> 16));
+		if((a.ext & EXT_MOVING_BOUNDARIES) && (flB & TYPE_BO) == TYPE_MS) moving_boundaries<Q>(a, make_site(xa + 1u, y, z, a.Nx, a.Ny, a.Nz), f);
 		collide_cell<Q, TRT, EXT, false, shared_division(ST, EXT), shared_pair_difference(Q, EXT, BUF)>(a, n + 1u, flB & TYPE_BO, f, nullptr);
 #pragma unroll
 		for(int i = 0; i < Q; i++) P[i] = S::encode_high(f[i], P[i]); // (code << 16) | (P & 0xFFFF)

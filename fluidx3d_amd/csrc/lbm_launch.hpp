@@ -228,15 +228,23 @@ constexpr bool tune_offsets32(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
 // EQUILIBRIUM_BOUNDARIES and + FORCE_FIELD +8 to +13 %; TRT none +1.9 / +4.1 %,
 // EQUILIBRIUM_BOUNDARIES +3.6 / +0.3, + FORCE_FIELD +3.9 / +0.3, porous +1.5 / +7.3; SRT
 // VOLUME_FORCE +1.6 / -0.7 and SRT porous -0.3 / +3.7 (each for the storage it gains on).
-// TRT VOLUME_FORCE (-1.3 / +0.1), the all-extension kernels (SRT -7 to -8 %; and the pair
-// kernel has no MOVING_BOUNDARIES) and D3Q27 (133-156 VGPRs, -13 to +0.3 %) keep one cell per lane.
+// TRT VOLUME_FORCE (-1.3 / +0.1), the all-extension kernels (SRT -7 to -8 %) and D3Q27
+// (133-156 VGPRs, -13 to +0.3 %) keep one cell per lane.  The kernels with SUBGRID, against
+// one cell per lane through buffer instructions (128^3, 256^3, 512x256x256): SRT +9 to +10 %
+// FP16S, +3 to +7 FP16C (with EQUILIBRIUM_BOUNDARIES +1 to +10, -1 to +6), TRT +3 to +6 FP16S,
+// -5.5 to +1 FP16C; with MOVING_BOUNDARIES and SUBGRID the same within 1 %, with
+// MOVING_BOUNDARIES alone +5 to +13 for every one, so that TRT FP16C leaves only SUBGRID out
+// (pair_extensions).
 constexpr bool tune_pairs(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
 	constexpr uint32_t POROUS = EXT_VOLUME_FORCE | EXT_POROSITY | EXT_PRECISE_DENSITY;
-	if(Q != 19 || ST == ST_FP32 || (EXT & (EXT_MOVING_BOUNDARIES | EXT_SUBGRID)) != 0u) return false;
+	if(Q != 19 || ST == ST_FP32 || EXT == EXT_ALL) return false;
+	if(EXT == EXT_LES) return !TRT || ST == ST_FP16S;
+	if(EXT == EXT_LES_MOVING) return true;
 	if(EXT == EXT_VOLUME_FORCE) return !TRT && ST == ST_FP16S;
 	if(EXT == POROUS) return TRT || ST == ST_FP16C;
 	return EXT == 0u || EXT == EXT_EQUILIBRIUM_BOUNDARIES || EXT == (EXT_EQUILIBRIUM_BOUNDARIES | EXT_FORCE_FIELD);
 }
+inline bool pair_extensions(uint32_t storage, bool trt, uint32_t ext) { return !(trt && storage == ST_FP16C && (ext & EXT_SUBGRID)); }
 // Buffer instructions on the row grid (load_raw's BUF: one buffer resource, scalar slot and
 // row offsets, three lane offsets) for the 16-bit kernels that keep one cell per lane: their
 // vector registers fall from 59-100 to 43-85 (the C3-type D3Q27 TRT FP16C kernel with
@@ -251,10 +259,11 @@ constexpr bool tune_pairs(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
 // (FP16C) +2.4.  Not taken: D3Q27 SRT none (-3.3 / -3.7), D3Q27 SRT VOLUME_FORCE FP16S,
 // D3Q19 SRT all extensions (-2.2 / -1.5), every FP32 kernel (-9 to +1 %: they wait on HBM),
 // and the D3Q19 kernels of tune_pairs (two cells per lane; on rows of half a wave they keep
-// the one-cell form they had).
+// the one-cell form they had, which for the SUBGRID and MOVING_BOUNDARIES subsets is this one).
 constexpr bool tune_buffer(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
 	if(ST == ST_FP32) return false;
 	if(Q == 27) return TRT || (EXT != 0u && !(EXT == EXT_VOLUME_FORCE && ST == ST_FP16S));
+	if(EXT == EXT_LES || EXT == EXT_LES_MOVING) return true;
 	return !tune_pairs(Q, ST, TRT, EXT) && (TRT || EXT != EXT_ALL);
 }
 // The two-cells-per-lane kernel through buffer instructions (its BUF): its stores no longer
