@@ -3,7 +3,6 @@
 // device/buffer/kernel layer of the reference (src/opencl.hpp:284-692).
 #include <hip/hip_runtime.h>
 #include <cstdio>
-#include <cstdlib>
 #include <cstring>
 #include <cmath>
 #include <string>
@@ -41,10 +40,12 @@ struct fx_ctx {
 	hipStream_t stream = nullptr;
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
 	const fx::LbmKernels* k = nullptr;
+	fx::Divisor by_Nx, by_Ny;
 	fx::LaunchShape shape{};    // one lane per cell: every kernel but stream_collide
 	fx::LaunchShape shape_sc{}; // stream_collide (residency cap, XCD-mapped grid)
 	fx::LaunchShape shape_uf{};  // update_fields
-	fx::LaunchShape shape_adj{}; // record pass and adjoint step (XCD-mapped grid)
+	fx::LaunchShape shape_rec{}; // the adjoint's record pass
+	fx::LaunchShape shape_adj{}; // adjoint step (XCD-mapped grid)
 	double* partial = nullptr; // reduction partials (device)
 	uint64_t partial_cap = 0;  // in doubles
 	double* result = nullptr;  // 4 doubles (device)
@@ -230,6 +231,7 @@ fx::LbmArgs make_args(const fx_ctx* ctx, const void* fi, const float* rho, const
 	a.Nx = ctx->cfg.Nx; a.Ny = ctx->cfg.Ny; a.Nz = ctx->cfg.Nz;
 	a.ext = ctx->cfg.extensions;
 	a.odd = (uint32_t)(t & 1ull);
+	a.by_Nx = ctx->by_Nx; a.by_Ny = ctx->by_Ny;
 	a.xchunks = 0u; // set by the stream_collide launcher from its shape
 	a.reverse = 0u;
 	a.w = ctx->cfg.w;
@@ -577,6 +579,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	ctx->device = device;
 	ctx->cfg = *cfg;
 	ctx->N = N;
+	ctx->by_Nx = fx::Divisor(cfg->Nx); ctx->by_Ny = fx::Divisor(cfg->Ny);
 	ctx->k = fx::select_kernels(cfg->velocity_set, cfg->storage, cfg->collision == FX_TRT, cfg->extensions);
 	ctx->shape = fx::lattice_shape(cfg->Nx, cfg->Ny, cfg->Nz);
 	ctx->shape_sc = fx::stream_shape(cfg->Nx, cfg->Ny, cfg->Nz, ctx->k->stream_collide_xcd_map);
@@ -599,16 +602,27 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	ctx->shape_uf = fx::use_linear_grid(*ctx->k, cfg->Nx, eb, N, cfg->velocity_set) ? fx::linear_shape(N, ctx->k->stream_collide_linear_xcd)
 	                                                                               : fx::stream_shape(cfg->Nx, cfg->Ny, cfg->Nz, true);
 	ctx->shape_uf.buf = N * cfg->velocity_set * eb <= 0xFFFFFFFFull;
+	ctx->shape_rec = ctx->shape_adj;
+	const uint64_t ddf = N * cfg->velocity_set * eb;
+	if(ddf <= fx::CACHED_BYTES) {
+		if(ddf > fx::L2_BYTES && ctx->k->stream_collide_cached_pairs && fx::pair_rows(cfg->Nx) && fx::pair_extensions(cfg->storage, cfg->collision == FX_TRT, cfg->extensions)) {
+			ctx->shape_sc = fx::pair_shape(cfg->Nx, cfg->Ny, cfg->Nz);
+			ctx->shape_sc.cached = true;
+		} else ctx->shape_sc = fx::slab_shape(N);
+		ctx->shape_rec = fx::slab_shape(N);
+		if(ddf + 17u * N <= fx::CACHED_BYTES) ctx->shape_uf = fx::slab_shape(N); // the DDFs and what update_fields writes
+	}
 	ctx->shape_sc.alternate = N * cfg->velocity_set * eb >= fx::ALTERNATE_ORDER_BYTES;
-	ctx->shape_adj.alternate = ctx->shape_sc.alternate;
-	const uint32_t cap = ctx->k->stream_collide_waves_cap;
+	ctx->shape_adj.alternate = ctx->shape_rec.alternate = ctx->shape_sc.alternate;
+	const uint32_t cap = ctx->shape_sc.cached ? 0u : ctx->k->stream_collide_waves_cap;
 	hipError_t e = hipSetDevice(device);
 	if(e == hipSuccess) {
 		hipDeviceProp_t prop;
 		e = hipGetDeviceProperties(&prop, device);
 		// k_two_steps has 32-bit byte offsets within a plane
 		if(e == hipSuccess && ctx->k->two_steps && (uint64_t)cfg->Nx * cfg->Ny * eb <= 0xFFFFFFFFull) {
-			const fx::TwoStepShape two = fx::two_step_shape(cfg->Nx, cfg->Ny, cfg->Nz, (uint32_t)prop.multiProcessorCount);
+			fx::TwoStepShape two = fx::two_step_shape(cfg->Nx, cfg->Ny, cfg->Nz, (uint32_t)prop.multiProcessorCount);
+			two.cached = 2u * ddf <= fx::CACHED_BYTES;
 			if(fx::two_steps_pay(two, cfg->Nx, cfg->Ny, cfg->Nz, cfg->velocity_set, cfg->collision == FX_TRT, cfg->extensions)) ctx->shape_two = two;
 		}
 		if(e == hipSuccess && cap)
@@ -937,7 +951,7 @@ int fx_lbm_stream_collide_record(fx_ctx* ctx, void* fi, float* rho, float* u, co
 	if(ctx->cfg.extensions & (FX_MOVING_BOUNDARIES | FX_SUBGRID))
 		return fail(FX_ERR_CONFIG, "the adjoint does not differentiate MOVING_BOUNDARIES or SUBGRID");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	ctx->k->stream_collide_record(make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), ctx->shape_adj, ctx->stream, moments);
+	ctx->k->stream_collide_record(make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), ctx->shape_rec, ctx->stream, moments);
 	return check_launch("stream_collide_record");
 }
 
@@ -1044,7 +1058,7 @@ int fx_lbm_backward(fx_ctx* ctx, fx_adjoint* adj, const float* rho, const float*
 		FX_HIP(hipMemcpyAsync(adj->work_fi, adj->ckpt + s * adj->fi_bytes, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
 		for(uint64_t t = ts; t < te; t++) {
 			a.odd = (uint32_t)(t & 1u);
-			ctx->k->stream_collide_record(a, ctx->shape_adj, ctx->stream, adj->moments + (t - ts) * 4u * N);
+			ctx->k->stream_collide_record(a, ctx->shape_rec, ctx->stream, adj->moments + (t - ts) * 4u * N);
 		}
 		for(uint64_t t = te; t-- > ts;) {
 			fx::AdjointArgs g = adjoint_args(ctx, adj->lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, adj->moments + (t - ts) * 4u * N,

@@ -33,6 +33,20 @@ constexpr float THIRD = 0.33333334f; // src/kernel.cpp:1093-1099
 constexpr float SMAGORINSKY = 0.76421222f; // 18*sqrt(2)*(C*Delta)^2, src/kernel.cpp:1591
 
 // Kernel arguments, passed by value (kernarg segment -> scalar registers).
+// n / d for n below 2^31 and d from 1 to 2^31 as a multiplication (Granlund and Montgomery, "Division
+// by invariant integers using multiplication", 1994): m = ceil(2^(31+l) / d) fits 32 bits for
+// l = ceil(log2 d), and n * (m*d - 2^(31+l)) < 2^(31+l).
+struct Divisor {
+	uint32_t m = 0, shift = 0;
+	Divisor() = default;
+	explicit Divisor(uint32_t d) {
+		uint32_t l = 0;
+		while(l < 31u && (1u << l) < d) l++;
+		m = d <= 1u ? 0u : (uint32_t)(((1ull << (31u + l)) + d - 1u) / d);
+		shift = d <= 1u ? 0u : l - 1u;
+	}
+	__host__ __device__ uint32_t quotient(uint32_t n) const { return m ? (uint32_t)(((uint64_t)n * m) >> 32) >> shift : n; }
+};
 struct LbmArgs {
 	void* fi;
 	float* rho;
@@ -47,6 +61,7 @@ struct LbmArgs {
 	float w;
 	float wm;       // TRT antisymmetric rate trt_minus_rate(w), formed once by the host
 	float fx, fy, fz;
+	Divisor by_Nx, by_Ny; // for the cached kernels (cell_coords)
 	uint32_t xchunks; // stream_collide on a 1-D XCD-mapped grid: x chunks per row (0: 3-D grid)
 	uint32_t reverse; // stream_collide takes the blocks in reverse order (block_coords, cell_coords)
 };
@@ -437,6 +452,8 @@ __device__ __forceinline__ Site make_site(uint32_t x, uint32_t y, uint32_t z, ui
 // up); FP32 -2.3 to +1 %, not taken.
 // O32: the same 32-bit offsets on the row grid (the row grid's access rule), for lattices
 // whose slots are below 4 GiB; tune_offsets32 selects the kernels that gain from it.
+// CACHED: no non-temporal access at any slot, for lattices that stay in the caches from one
+// step to the next (CACHED_BYTES).
 template<int Q, uint32_t ST> constexpr bool slot_offsets32(bool SC) { return SC && ST != ST_FP32; }
 // BUF: the row grid through buffer instructions, for a DDF array below 4 GiB.  The address
 // of every access is the array's base (a buffer resource in scalar registers) plus a scalar
@@ -468,7 +485,15 @@ template<uint32_t ST> __device__ __forceinline__ typename Storage<ST>::E stored(
 	if constexpr(ST == ST_FP32) return x;
 	else return Storage<ST>::encode(x);
 }
-template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false>
+template<uint32_t ST, bool CACHED> __device__ __forceinline__ typename Storage<ST>::E raw_elem(const typename Storage<ST>::E* p, uint32_t o) {
+	if constexpr(CACHED) return Storage<ST>::raw_cached(p, o);
+	else return Storage<ST>::raw(p, o);
+}
+template<uint32_t ST, bool CACHED> __device__ __forceinline__ void store_elem(typename Storage<ST>::E* p, uint32_t o, float x) {
+	if constexpr(CACHED) Storage<ST>::store_cached(p, o, x);
+	else Storage<ST>::store(p, o, x);
+}
+template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false, bool CACHED = false>
 __device__ __forceinline__ void load_raw(const typename Storage<ST>::E* fi, uint64_t N, const Site& s, uint32_t odd, typename Storage<ST>::E* r) {
 	typedef Storage<ST> S;
 	if constexpr(BUF && SC) { // the cell-linear grid: rows per lane, every shifted slot cached
@@ -476,11 +501,11 @@ __device__ __forceinline__ void load_raw(const typename Storage<ST>::E* fi, uint
 		constexpr uint32_t eb = sizeof(E);
 		const __amdgpu_buffer_rsrc_t rs = ddf_buffer(fi);
 		const uint32_t slot = (uint32_t)N * eb, c = ((uint32_t)s.R[4] + s.x) * eb;
-		r[0] = buffer_elem<E, true>(rs, c, 0u);
+		r[0] = buffer_elem<E, !CACHED>(rs, c, 0u);
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint32_t sa = odd ? (uint32_t)i : (uint32_t)(i + 1), sb = odd ? (uint32_t)(i + 1) : (uint32_t)i;
-			r[i] = buffer_elem<E, true>(rs, c, sa * slot);
+			r[i] = buffer_elem<E, !CACHED>(rs, c, sa * slot);
 			const uint32_t o = ((uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) + s.X[VS<Q>::cx[i] + 1]) * eb;
 			r[i + 1] = buffer_elem<E, false>(rs, o, sb * slot);
 		}
@@ -488,56 +513,56 @@ __device__ __forceinline__ void load_raw(const typename Storage<ST>::E* fi, uint
 	} else if constexpr(BUF) {
 		typedef typename Storage<ST>::E E;
 		constexpr uint32_t eb = sizeof(E);
-		constexpr bool shifted_nt = ST == ST_FP32 && Q == 19; // x-shifted loads: raw_shifted's rule
+		constexpr bool shifted_nt = ST == ST_FP32 && Q == 19 && !CACHED; // x-shifted loads: raw_shifted's rule
 		const __amdgpu_buffer_rsrc_t rs = ddf_buffer(fi);
 		const uint32_t slot = (uint32_t)N * eb, n0 = (uint32_t)s.R[4] * eb;
 		const uint32_t v[3] = {s.X[0] * eb, s.x * eb, s.X[2] * eb};
-		r[0] = buffer_elem<E, true>(rs, v[1], n0);
+		r[0] = buffer_elem<E, !CACHED>(rs, v[1], n0);
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint32_t sa = odd ? (uint32_t)i : (uint32_t)(i + 1), sb = odd ? (uint32_t)(i + 1) : (uint32_t)i;
-			r[i] = buffer_elem<E, true>(rs, v[1], sa * slot + n0);
+			r[i] = buffer_elem<E, !CACHED>(rs, v[1], sa * slot + n0);
 			const uint32_t ob = sb * slot + (uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) * eb;
 			if(VS<Q>::cx[i] != 0) r[i + 1] = buffer_elem<E, shifted_nt>(rs, v[VS<Q>::cx[i] + 1], ob);
-			else r[i + 1] = buffer_elem<E, true>(rs, v[1], ob);
+			else r[i + 1] = buffer_elem<E, !CACHED>(rs, v[1], ob);
 		}
 		return;
 	}
 	if constexpr(O32 || slot_offsets32<Q, ST>(SC)) {
 		const uint32_t c = (uint32_t)s.R[4] + s.x; // the cell's index
-		r[0] = S::raw(fi, c);
+		r[0] = raw_elem<ST, CACHED>(fi, c);
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint64_t sa = odd ? (uint64_t)i : (uint64_t)(i + 1);
 			const uint64_t sb = odd ? (uint64_t)(i + 1) : (uint64_t)i;
-			r[i] = S::raw(fi + sa * N, c);
+			r[i] = raw_elem<ST, CACHED>(fi + sa * N, c);
 			const uint32_t o = (uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) + s.X[VS<Q>::cx[i] + 1];
 			if(SC || VS<Q>::cx[i] != 0) r[i + 1] = S::raw_cached(fi + sb * N, o);
-			else r[i + 1] = S::raw(fi + sb * N, o);
+			else r[i + 1] = raw_elem<ST, CACHED>(fi + sb * N, o);
 		}
 		return;
 	}
 	const uint64_t n0 = s.R[4];
-	r[0] = S::raw(row_base<U>(fi + n0), s.x);
+	r[0] = raw_elem<ST, CACHED>(row_base<U>(fi + n0), s.x);
 #pragma unroll
 	for(int i = 1; i < Q; i += 2) {
 		const uint64_t sa = odd ? (uint64_t)i : (uint64_t)(i + 1);
 		const uint64_t sb = odd ? (uint64_t)(i + 1) : (uint64_t)i;
-		r[i] = S::raw(row_base<U>(fi + sa * N + n0), s.x);
+		r[i] = raw_elem<ST, CACHED>(row_base<U>(fi + sa * N + n0), s.x);
 		const typename Storage<ST>::E* pb = row_base<U>(fi + sb * N + s.row(VS<Q>::cy[i], VS<Q>::cz[i]));
 		const uint32_t xb = s.X[VS<Q>::cx[i] + 1];
 		if(SC) r[i + 1] = S::raw_cached(pb, xb);
-		else r[i + 1] = VS<Q>::cx[i] != 0 ? S::template raw_shifted<Q>(pb, xb) : S::raw(pb, xb);
+		else r[i + 1] = VS<Q>::cx[i] != 0 && !CACHED ? S::template raw_shifted<Q>(pb, xb) : raw_elem<ST, CACHED>(pb, xb);
 	}
 }
-template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false>
+template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false, bool CACHED = false>
 __device__ __forceinline__ void load_f(const typename Storage<ST>::E* fi, uint64_t N, const Site& s, uint32_t odd, float* f) {
 	typename Storage<ST>::E r[Q];
-	load_raw<Q, ST, U, SC, O32, BUF>(fi, N, s, odd, r);
+	load_raw<Q, ST, U, SC, O32, BUF, CACHED>(fi, N, s, odd, r);
 #pragma unroll
 	for(int i = 0; i < Q; i++) f[i] = Storage<ST>::decode(r[i]);
 }
-template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false>
+template<int Q, uint32_t ST, bool U = false, bool SC = false, bool O32 = false, bool BUF = false, bool CACHED = false>
 __device__ __forceinline__ void store_f(typename Storage<ST>::E* fi, uint64_t N, const Site& s, uint32_t odd, const float* f) {
 	typedef Storage<ST> S;
 	if constexpr(BUF && SC) {
@@ -545,13 +570,13 @@ __device__ __forceinline__ void store_f(typename Storage<ST>::E* fi, uint64_t N,
 		constexpr uint32_t eb = sizeof(E);
 		const __amdgpu_buffer_rsrc_t rs = ddf_buffer(fi);
 		const uint32_t slot = (uint32_t)N * eb, c = ((uint32_t)s.R[4] + s.x) * eb;
-		buffer_elem<E, true>(rs, c, 0u, stored<ST>(f[0]));
+		buffer_elem<E, !CACHED>(rs, c, 0u, stored<ST>(f[0]));
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint32_t sa = odd ? (uint32_t)i : (uint32_t)(i + 1), sb = odd ? (uint32_t)(i + 1) : (uint32_t)i;
 			const uint32_t o = ((uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) + s.X[VS<Q>::cx[i] + 1]) * eb;
 			buffer_elem<E, false>(rs, o, sb * slot, stored<ST>(f[i]));
-			buffer_elem<E, true>(rs, c, sa * slot, stored<ST>(f[i + 1]));
+			buffer_elem<E, !CACHED>(rs, c, sa * slot, stored<ST>(f[i + 1]));
 		}
 		return;
 	} else if constexpr(BUF) {
@@ -560,33 +585,33 @@ __device__ __forceinline__ void store_f(typename Storage<ST>::E* fi, uint64_t N,
 		const __amdgpu_buffer_rsrc_t rs = ddf_buffer(fi);
 		const uint32_t slot = (uint32_t)N * eb, n0 = (uint32_t)s.R[4] * eb;
 		const uint32_t v[3] = {s.X[0] * eb, s.x * eb, s.X[2] * eb};
-		buffer_elem<E, true>(rs, v[1], n0, stored<ST>(f[0]));
+		buffer_elem<E, !CACHED>(rs, v[1], n0, stored<ST>(f[0]));
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint32_t sa = odd ? (uint32_t)i : (uint32_t)(i + 1), sb = odd ? (uint32_t)(i + 1) : (uint32_t)i;
 			const uint32_t ob = sb * slot + (uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) * eb;
 			if(VS<Q>::cx[i] != 0) buffer_elem<E, false>(rs, v[VS<Q>::cx[i] + 1], ob, stored<ST>(f[i]));
-			else buffer_elem<E, true>(rs, v[1], ob, stored<ST>(f[i]));
-			buffer_elem<E, true>(rs, v[1], sa * slot + n0, stored<ST>(f[i + 1]));
+			else buffer_elem<E, !CACHED>(rs, v[1], ob, stored<ST>(f[i]));
+			buffer_elem<E, !CACHED>(rs, v[1], sa * slot + n0, stored<ST>(f[i + 1]));
 		}
 		return;
 	}
 	if constexpr(O32 || slot_offsets32<Q, ST>(SC)) {
 		const uint32_t c = (uint32_t)s.R[4] + s.x;
-		S::store(fi, c, f[0]);
+		store_elem<ST, CACHED>(fi, c, f[0]);
 #pragma unroll
 		for(int i = 1; i < Q; i += 2) {
 			const uint64_t sa = odd ? (uint64_t)i : (uint64_t)(i + 1);
 			const uint64_t sb = odd ? (uint64_t)(i + 1) : (uint64_t)i;
 			const uint32_t o = (uint32_t)s.row(VS<Q>::cy[i], VS<Q>::cz[i]) + s.X[VS<Q>::cx[i] + 1];
 			if(SC || VS<Q>::cx[i] != 0) S::store_cached(fi + sb * N, o, f[i]);
-			else S::store(fi + sb * N, o, f[i]);
-			S::store(fi + sa * N, c, f[i + 1]);
+			else store_elem<ST, CACHED>(fi + sb * N, o, f[i]);
+			store_elem<ST, CACHED>(fi + sa * N, c, f[i + 1]);
 		}
 		return;
 	}
 	const uint64_t n0 = s.R[4];
-	S::store(row_base<U>(fi + n0), s.x, f[0]);
+	store_elem<ST, CACHED>(row_base<U>(fi + n0), s.x, f[0]);
 #pragma unroll
 	for(int i = 1; i < Q; i += 2) {
 		const uint64_t sa = odd ? (uint64_t)i : (uint64_t)(i + 1);
@@ -595,8 +620,8 @@ __device__ __forceinline__ void store_f(typename Storage<ST>::E* fi, uint64_t N,
 		const uint32_t xb = s.X[VS<Q>::cx[i] + 1];
 		if(VS<Q>::cx[i] != 0) S::template store_shifted<Q>(pb, xb, f[i]);
 		else if(SC) S::store_cached(pb, xb, f[i]);
-		else S::store(pb, xb, f[i]);
-		S::store(row_base<U>(fi + sa * N + n0), s.x, f[i + 1]);
+		else store_elem<ST, CACHED>(pb, xb, f[i]);
+		store_elem<ST, CACHED>(row_base<U>(fi + sa * N + n0), s.x, f[i + 1]);
 	}
 }
 
@@ -803,6 +828,11 @@ __device__ __forceinline__ void collide_pairs(float w, float wm, bool vf, bool i
 		}
 	}
 }
+// The adjoint's moments are written once and read once, a segment of steps later: from
+// MOMENTS_STREAM cells on past the caches (non-temporal), which then keep the DDFs and the
+// adjoint populations.  Backward sweep of 64 steps, us per step: 150x150x130 231 -> 205, 128^3 FP32
+// 135.2 -> 132.6, D3Q27 TRT 212 -> 197; 128x64x64 39.8 -> 40.2, 128x96x96 FP16S 67.5 -> 69.9.
+constexpr uint64_t MOMENTS_STREAM = 1ull << 21;
 // SD: u = j/rho and 0.5/rho through SharedDivisor; only where shared_division allows it.
 // SHARE: the whole-array TRT collision forms each opposite pair's equilibrium difference
 // once (shared_pair_difference).
@@ -819,7 +849,12 @@ __device__ __forceinline__ void collide_cell(const LbmArgs& a, uint64_t n, uint3
 			for(int i = 1; i < Q; i++) rhom1 += fhn[i];
 		} else rhom1 = rhon - 1.0f;
 		if constexpr(RECORD) { // pre-collision moments for the adjoint sweep
-			moments[n] = rhon; moments[a.N + n] = jx; moments[2ull * a.N + n] = jy; moments[3ull * a.N + n] = jz;
+			if(a.N >= MOMENTS_STREAM) {
+				__builtin_nontemporal_store(rhon, moments + n);
+				__builtin_nontemporal_store(jx, moments + a.N + n); __builtin_nontemporal_store(jy, moments + 2ull * a.N + n); __builtin_nontemporal_store(jz, moments + 3ull * a.N + n);
+			} else {
+				moments[n] = rhon; moments[a.N + n] = jx; moments[2ull * a.N + n] = jy; moments[3ull * a.N + n] = jz;
+			}
 		}
 		if constexpr(SD) {
 			const SharedDivisor dv(rhon);
@@ -927,6 +962,10 @@ template<bool XCD> __device__ __forceinline__ bool block_coords(const LbmArgs& a
 	y = row - z * a.Ny;
 	return true;
 }
+// Segment of block L where each XCD takes one eighth of the lattice, a slab of consecutive
+// segments (blocks: a multiple of 8), so that the lines a step leaves in an L2 are the ones
+// that its XCD reads in the next step, except at the slabs' ends.  A permutation.
+__host__ __device__ inline uint64_t slab_segment(uint64_t L, uint64_t blocks) { return (L & 7u) * (blocks >> 3) + (L >> 3); }
 // Segment (block of consecutive cells) of block L on the cell-linear grid.  The hardware
 // hands consecutive blocks to the 8 XCDs in turn; with xcd and a grid of whole groups of
 // 64 blocks, group g's block 8j + k takes segment 64g + 8k + j, so each XCD runs 8
@@ -940,9 +979,20 @@ __host__ __device__ inline uint64_t linear_segment(uint64_t L, uint64_t blocks, 
 // linear_segment(L) of blockDim.x consecutive cells of the whole lattice, rows and planes
 // crossed wherever they end (every wave starts on a multiple of 64 cells, so its unshifted
 // slot accesses are whole 128-byte lines whatever Nx is); XCD there selects the XCD-aware
-// segment order.  Otherwise the row grid of block_coords.  False for lanes past the lattice.
-template<bool XCD, bool LIN> __device__ __forceinline__ bool cell_coords(const LbmArgs& a, uint32_t& x, uint32_t& y, uint32_t& z) {
-	if constexpr(LIN) {
+// segment order and CACHED the slabs of slab_segment.  Otherwise the row grid of block_coords.  False for lanes past the lattice.
+template<bool XCD, bool LIN, bool CACHED = false> __device__ __forceinline__ bool cell_coords(const LbmArgs& a, uint32_t& x, uint32_t& y, uint32_t& z) {
+	if constexpr(LIN && CACHED) { // a small lattice: 32-bit cell indices, short of 2^31
+		// by_Nx, by_Ny instead of a 64-bit division, which every wave waits for before its first
+		// load: 24x16x12 FP32 4.05 -> 3.33 us, FP16S 4.13 -> 3.44, 64^3 6.55 -> 5.98, 17x300x100 FP16S
+		// 9.4 -> 8.9, from 100^3 on the same within 2 %
+		const uint32_t n = (uint32_t)slab_segment(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+		if(n >= (uint32_t)a.N) return false;
+		const uint32_t r = a.by_Nx.quotient(n);
+		x = n - r * a.Nx;
+		z = a.by_Ny.quotient(r);
+		y = r - z * a.Ny;
+		return true;
+	} else if constexpr(LIN) {
 		const uint32_t L = a.reverse ? gridDim.x - 1u - blockIdx.x : blockIdx.x;
 		const uint64_t c0 = linear_segment(L, gridDim.x, XCD) * blockDim.x; // first cell of the block
 		if(c0 + threadIdx.x >= a.N) return false;
@@ -964,12 +1014,12 @@ template<bool XCD, bool LIN> __device__ __forceinline__ bool cell_coords(const L
 	}
 }
 // One lane per cell.
-template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool RECORD, bool XCD, bool LIN, bool O32 = false, bool BUF = false>
+template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool RECORD, bool XCD, bool LIN, bool O32 = false, bool BUF = false, bool CACHED = false>
 __device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments) {
 	a.ext &= EXT;
 	if constexpr(constant_vf_mask<TRT>(Q, ST, EXT, LIN)) a.ext = EXT_VOLUME_FORCE;
 	uint32_t x, y, z;
-	if(!cell_coords<XCD, LIN>(a, x, y, z)) return;
+	if(!cell_coords<XCD, LIN, CACHED>(a, x, y, z)) return;
 	constexpr bool U = !LIN && uniform_rows<TRT>(Q, ST, EXT); // rows are per lane on the cell-linear grid
 	const Site s = make_site(x, y, z, a.Nx, a.Ny, a.Nz);
 	const uint64_t n = s.n();
@@ -984,24 +1034,24 @@ __device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments) {
 		// convert each 16-bit value right after its load and wait for it, one at a time
 		E r[Q];
 		if constexpr(load_priority<TRT>(EXT)) __builtin_amdgcn_s_setprio(1);
-		load_raw<Q, ST, U, LIN, O32, BUF>(fi, a.N, s, a.odd, r);
+		load_raw<Q, ST, U, LIN, O32, BUF, CACHED>(fi, a.N, s, a.odd, r);
 		__builtin_amdgcn_sched_barrier(0);
 		if constexpr(load_priority<TRT>(EXT)) __builtin_amdgcn_s_setprio(0);
 #pragma unroll
 		for(int i = 0; i < Q; i++) f[i] = Storage<ST>::decode(r[i]);
 	} else {
-		load_f<Q, ST, U, LIN, O32, BUF>(fi, a.N, s, a.odd, f);
+		load_f<Q, ST, U, LIN, O32, BUF, CACHED>(fi, a.N, s, a.odd, f);
 	}
 	if((a.ext & EXT_MOVING_BOUNDARIES) && bo == TYPE_MS) moving_boundaries<Q>(a, s, f);
 	collide_cell<Q, TRT, EXT, RECORD, shared_division(ST, EXT), shared_pair_difference(Q, EXT, BUF)>(a, n, bo, f, moments);
-	store_f<Q, ST, U, LIN, O32, BUF>(fi, a.N, s, a.odd, f);
+	store_f<Q, ST, U, LIN, O32, BUF, CACHED>(fi, a.N, s, a.odd, f);
 }
 // XCD: the kernel may run on the 1-D XCD-mapped grid (a.xchunks > 0); false compiles the
 // mapping out.  LIN: the cell-linear grid (cell_coords), for lattices whose rows do not
 // start on 128-byte lines.
-template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false, bool O32 = false, bool BUF = false>
+template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false, bool O32 = false, bool BUF = false, bool CACHED = false>
 __global__ __launch_bounds__(BLOCK) void k_stream_collide(LbmArgs a) {
-	stream_collide_cell<Q, ST, TRT, EXT, false, XCD, LIN, O32, BUF>(a, nullptr);
+	stream_collide_cell<Q, ST, TRT, EXT, false, XCD, LIN, O32, BUF, CACHED>(a, nullptr);
 }
 // stream_collide with two adjacent cells per lane, for the 16-bit formats on rows of whole
 // waves of lanes (Nx a multiple of 128, pair_rows).  A wave takes the 128 cells c0 .. c0+127
@@ -1043,7 +1093,7 @@ __device__ __forceinline__ gcode* code_at(gcode* p, uint32_t x) { return (gcode*
 __device__ __forceinline__ gword* word_at(gcode* p, uint32_t x) { return (gword*)code_at(p, x); } // x even
 // BUF: every access through buffer instructions (load_raw's BUF; a DDF array below 4 GiB):
 // no 64-bit store addresses rebuilt in vector registers after the collision.
-template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool BUF = false>
+template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool BUF = false, bool CACHED = false>
 __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 	static_assert(ST != ST_FP32, "16-bit codes only");
 	a.ext &= EXT;
@@ -1069,11 +1119,13 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 	const uint64_t N = a.N, n0 = s.R[4];
 	// a slot row's first element (uniform): its word at xa, its codes at q
 	const auto word_load = [&](uint64_t row) -> uint32_t {
-		if constexpr(BUF) return buffer_elem<uint32_t, true>(ddf_buffer(fi), xa * 2u, (uint32_t)row * 2u);
+		if constexpr(BUF) return buffer_elem<uint32_t, !CACHED>(ddf_buffer(fi), xa * 2u, (uint32_t)row * 2u);
+		else if constexpr(CACHED) return *word_at(global_row(fi + row), xa);
 		else return __builtin_nontemporal_load(word_at(global_row(fi + row), xa));
 	};
 	const auto word_store = [&](uint64_t row, uint32_t w) {
-		if constexpr(BUF) buffer_elem<uint32_t, true>(ddf_buffer(fi), xa * 2u, (uint32_t)row * 2u, w);
+		if constexpr(BUF) buffer_elem<uint32_t, !CACHED>(ddf_buffer(fi), xa * 2u, (uint32_t)row * 2u, w);
+		else if constexpr(CACHED) *word_at(global_row(fi + row), xa) = w;
 		else __builtin_nontemporal_store(w, word_at(global_row(fi + row), xa));
 	};
 	const auto code_load = [&](uint64_t row, uint32_t q) -> uint32_t {
@@ -1172,9 +1224,9 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 // moments[c*N+n], c = 0..3 (16 B/cell): what the adjoint step needs of the forward state.
 // EXT is the context's extension subset; MOVING_BOUNDARIES and SUBGRID are not
 // differentiated and compiled out.
-template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false>
+template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false, bool CACHED = false>
 __global__ __launch_bounds__(BLOCK) void k_stream_collide_record(LbmArgs a, float* moments) {
-	stream_collide_cell<Q, ST, TRT, EXT & ~(EXT_MOVING_BOUNDARIES | EXT_SUBGRID), true, XCD, LIN>(a, moments);
+	stream_collide_cell<Q, ST, TRT, EXT & ~(EXT_MOVING_BOUNDARIES | EXT_SUBGRID), true, XCD, LIN, false, false, CACHED>(a, moments);
 }
 
 // update_fields (src/kernel.cpp:1794-1870), on the grids of stream_collide (cell_coords).
@@ -1185,12 +1237,15 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_record(LbmArgs a, floa
 // 200^3 FP32 160 -> 106 us, FP16C 87 -> 70, 160x120x100 FP16S 25.7 -> 20.5, 201x75x99 FP32 31.8
 // -> 25.0.  BUF on the row grid: rows of several blocks, 384x192x192 FP16S 130 -> 121 and
 // D3Q27 FP16C 169 -> 155 (rows of one block: 256^3 D3Q19 -3 %, D3Q27 +7 %, 128^3 +5 to +11 %).
+// CACHED where the DDFs and the fields stay in the last-level cache: 128^3 FP32 36.4 -> 26.7,
+// 160x120x100 FP16S 20.5 -> 17.0, 64^3 FP32 5.4 -> 4.0, 24x16x12 4.4 -> 3.5 (192x192x160 FP16S, whose
+// fields do not fit, 54 -> 65).
 constexpr uint64_t UPDATE_FIELDS_STREAM = 1ull << 19;
-template<int Q, uint32_t ST, uint32_t EXT, bool XCD, bool LIN, bool BUF>
+template<int Q, uint32_t ST, uint32_t EXT, bool XCD, bool LIN, bool BUF, bool CACHED = false>
 __global__ __launch_bounds__(BLOCK) void k_update_fields(LbmArgs a) {
 	a.ext &= EXT;
 	uint32_t x, y, z;
-	if(!cell_coords<XCD, LIN>(a, x, y, z)) return;
+	if(!cell_coords<XCD, LIN, CACHED>(a, x, y, z)) return;
 	const Site s = make_site(x, y, z, a.Nx, a.Ny, a.Nz);
 	const uint64_t n = s.n();
 	const uint32_t flagsn = a.flags[n];
@@ -1198,7 +1253,7 @@ __global__ __launch_bounds__(BLOCK) void k_update_fields(LbmArgs a) {
 	if(bo == TYPE_S || (flagsn & TYPE_SU) == TYPE_G) return;
 	float fhn[Q];
 	typename Storage<ST>::E r[Q];
-	load_raw<Q, ST, false, LIN, false, BUF>((const typename Storage<ST>::E*)a.fi, a.N, s, a.odd, r);
+	load_raw<Q, ST, false, LIN, false, BUF, CACHED>((const typename Storage<ST>::E*)a.fi, a.N, s, a.odd, r);
 	if constexpr(ST == ST_FP16S) __builtin_amdgcn_sched_barrier(0); // every load before the first conversion
 #pragma unroll
 	for(int i = 0; i < Q; i++) fhn[i] = Storage<ST>::decode(r[i]);
@@ -1403,8 +1458,14 @@ __global__ __launch_bounds__(BLOCK) void k_adjoint_step(AdjointArgs g) {
 	float rho, u0x, u0y, u0z;
 	if(isE) { rho = a.rho[n]; u0x = a.u[n]; u0y = a.u[a.N + n]; u0z = a.u[2ull * a.N + n]; }
 	else {
-		rho = g.moments[n];
-		u0x = g.moments[a.N + n] / rho; u0y = g.moments[2ull * a.N + n] / rho; u0z = g.moments[3ull * a.N + n] / rho;
+		float jx, jy, jz;
+		if(a.N >= MOMENTS_STREAM) {
+			rho = __builtin_nontemporal_load(g.moments + n);
+			jx = __builtin_nontemporal_load(g.moments + a.N + n); jy = __builtin_nontemporal_load(g.moments + 2ull * a.N + n); jz = __builtin_nontemporal_load(g.moments + 3ull * a.N + n);
+		} else {
+			rho = g.moments[n]; jx = g.moments[a.N + n]; jy = g.moments[2ull * a.N + n]; jz = g.moments[3ull * a.N + n];
+		}
+		u0x = jx / rho; u0y = jy / rho; u0z = jz / rho;
 	}
 	float ubx = u0x, uby = u0y, ubz = u0z, k = 1.0f;
 	if(vf) {

@@ -11,6 +11,7 @@ struct LaunchShape {
 	size_t lds = 0;       // dynamic LDS reserved per block (occupancy limit), see occupancy_lds()
 	uint32_t xchunks = 0; // 1-D XCD-mapped grid with this many x chunks per row (see block_coords)
 	bool lin = false;     // cell-linear grid (cell_coords in lbm_device.hpp), see linear_shape
+	bool cached = false;  // the DDFs stay in the caches between steps (CACHED_BYTES)
 	bool pairs = false;   // two cells per lane (k_stream_collide_pair), see pair_shape
 	bool off32 = false;   // row grid with 32-bit slot offsets (O32 of load_raw/store_f)
 	bool buf = false;     // row grid through buffer instructions (BUF of load_raw/store_f)
@@ -40,6 +41,24 @@ inline LaunchShape linear_shape(uint64_t N, bool xcd) {
 	s.block = dim3(256, 1, 1);
 	s.grid = dim3((unsigned)blocks, 1, 1);
 	s.lin = true;
+	return s;
+}
+// Lattices whose DDFs stay in the last-level cache (256 MiB) from one step to the next: no
+// non-temporal accesses, which leave the lines out of it, and one slab of the lattice per XCD
+// (slab_segment; slab_shape, the cell-linear grid whether rows start on lines or not).  Bound
+// by that cache (7.0 TB/s in place, against 6.3 from HBM) and below L2_BYTES, all L2s together, by
+// the start of a launch.  fx_lbm_run, us per step before -> now: D3Q19 SRT FP16S 64^3 7.8 ->
+// 5.9, 128^3 30.8 -> 26.7 (two cells per lane), 160x120x100 31.1 -> 26.0, 192x192x160 88 -> 67;
+// FP32 24x16x12 4.3 -> 3.3, 64^3 7.6 (two steps per launch) -> 6.0, 141x140x139 78 (two) -> 63;
+// D3Q27 SRT FP16S 128^3 49.6 -> 37.5, TRT FP16C EQUILIBRIUM_BOUNDARIES + FORCE_FIELD 48.7 ->
+// 42.9.  Every kernel measured at 64^3 to 224 MiB gains, +1 to +56 %
+// (1024x16x8 FP32 -2 to -4).  The line: 160^3 D3Q27
+// TRT FP16C (211 MiB) +2 %, D3Q19 170x168x168 to 184x180x180 (174 to 216 MiB) +23 to +56 %;
+// 128x192x192 D3Q27 (243 MiB) -6 to +40 %, 192^3 FP16S (256 MiB) -9 %, 256x256x128 -14 %.
+constexpr uint64_t CACHED_BYTES = 224ull << 20, L2_BYTES = 32ull << 20;
+inline LaunchShape slab_shape(uint64_t N) {
+	LaunchShape s = linear_shape(N, true);
+	s.cached = true;
 	return s;
 }
 // Block of bx consecutive x cells of one row (bx = 64, 128 or 256); grid over (x chunk,
@@ -101,6 +120,7 @@ inline size_t occupancy_lds(uint32_t waves_per_simd, uint32_t block_threads, siz
 // planes; tiles of at most 128 x 5 columns, 64 x 13 on rows of at most 64 cells.
 struct TwoStepShape {
 	bool wide = false;
+	bool cached = false; // cached stores: both DDF arrays stay in the caches
 	uint32_t width = 0, height = 0, zlen = 0, tiles_x = 0, tiles_y = 0, tiles = 0, grid = 0; // grid 0: not used
 };
 constexpr uint32_t TWO_STEP_WIDE_X = 128u, TWO_STEP_WIDE_Y = 5u, TWO_STEP_NARROW_X = 64u, TWO_STEP_NARROW_Y = 13u;
@@ -167,6 +187,7 @@ struct LbmKernels {
 	bool stream_collide_pair_buffer;  // the same for k_stream_collide_pair
 	bool stream_collide_linear_buffer; // the same on the cell-linear grid
 	two_steps_fn two_steps;           // two time steps in one launch (k_two_steps), null where it does not pay
+	bool stream_collide_cached_pairs; // k_stream_collide_pair among the cached kernels
 };
 
 constexpr uint32_t EXT_ALL = EXT_VOLUME_FORCE | EXT_FORCE_FIELD | EXT_EQUILIBRIUM_BOUNDARIES | EXT_UPDATE_FIELDS | EXT_POROSITY |
@@ -245,6 +266,14 @@ constexpr bool tune_pairs(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
 	return EXT == 0u || EXT == EXT_EQUILIBRIUM_BOUNDARIES || EXT == (EXT_EQUILIBRIUM_BOUNDARIES | EXT_FORCE_FIELD);
 }
 inline bool pair_extensions(uint32_t storage, bool trt, uint32_t ext) { return !(trt && storage == ST_FP16C && (ext & EXT_SUBGRID)); }
+// Two cells per lane among the cached kernels (CACHED_BYTES; DDFs above L2_BYTES), against
+// slab_shape's one: tune_pairs' kernels -3 to +10 % (128x96x96 to 256x192x96; D3Q19 SRT FP16S
+// 128^3 27.3 -> 26.7 us, MOVING_BOUNDARIES + SUBGRID 30.5 -> 29.6, TRT FP16S porous 35.0 -> 33.7),
+// TRT FP16S VOLUME_FORCE +9 to +13 % (128^3 34.9 -> 30.9), TRT FP16C VOLUME_FORCE -2 to +2, SRT
+// FP16C VOLUME_FORCE -8 to +4.  Up to L2_BYTES (128x64x64) slab_shape is ahead by 2 to 18 %.
+constexpr bool tune_cached_pairs(int Q, uint32_t ST, bool TRT, uint32_t EXT) {
+	return tune_pairs(Q, ST, TRT, EXT) || (Q == 19 && ST == ST_FP16S && TRT && EXT == EXT_VOLUME_FORCE);
+}
 // Buffer instructions on the row grid (load_raw's BUF: one buffer resource, scalar slot and
 // row offsets, three lane offsets) for the 16-bit kernels that keep one cell per lane: their
 // vector registers fall from 59-100 to 43-85 (the C3-type D3Q27 TRT FP16C kernel with
@@ -330,17 +359,22 @@ constexpr bool tune_two_steps(int Q, uint32_t ST, bool TRT, uint32_t EXT) { retu
 // Lattices that gain.  The step t of a tile's border cells is taken twice and lanes beyond a
 // row's end idle, which costs the more the more arithmetic a cell has (weight: one each for
 // VOLUME_FORCE, POROSITY, TRT and D3Q27, two for SUBGRID), and a launch takes longer to start.
-// Lanes in use, Nx over the tiles' width: weight 0 to 2 gained 2 to 42 % at 55 to 63 % (140^3,
-// 72x128x128, 160^3) and -4 to +2 % at 51 % (130^3, 65^3); rows of at most 64 cells +1 % at
-// 38 % (Nx = 24), -16 % at 25 %; weight 3 and 4 -12 to +2 % at 56 to 78 % (160^3, 200^3), +6 to
-// +27 % above 90 %.  Cells: weight 0 -3 % at 32^3, +6 % at 40^3, +20 % at 48^3; weight 1 +10 to
-// +15 % at 64^3, weight 2 -2 to +4 % there and +3 to +22 % at 128x64x64, weight 3 and 4 -11 to
-// -3 % and +1 to +6 %.  One or two planes: 400x400x1 -20 %, x2 -5 %, x3 +1 %, x4 +4 %; rows of
-// one plane: 400x1x400 -20 %, 1000x1x300 -3 %, 1000x2x300 +37 %.
+// percent: lanes in use, Nx over the tiles' width.
+// DDFs above CACHED_BYTES: weight 0 to 2 gained 2 to 42 % at 55 to 63 % (160^3) and more above;
+// rows of at most 64 cells +1 % at 38 % (Nx = 24), -16 % at 25 %; weight 3 and 4 -12 to +2 % at
+// 56 to 78 % (160^3, 200^3), +6 to +27 % above 90 %.  One or two planes: 400x400x1 -20 %, x2
+// -5 %, x3 +1 %, x4 +4 %; rows of one plane: 400x1x400 -20 %, 1000x1x300 -3 %, 1000x2x300 +37 %.
+// Up to CACHED_BYTES single steps are faster (slab_shape).  At 100 % weight 0 and 1 still gain
+// 13 to 26 % (128x64x64, 128^3), weight 2 -2 to +13 %, weight 3 -4 to 0; at 87 % (112^3) 23 to 45 %,
+// 12 to 23 %, weight 2 +1 to +17 %; at 75 to 78 % with both DDF arrays in the cache +9 to +23 %
+// (96^3, 201x75x99), weight 2 -3 to -10 %, with one -5 % (201x75x99 D3Q27); at 56 to 62 % -40 to 0
+// (80^3, 144^3, 150x60x40).  Up to L2_BYTES -7 to -14 % (48^3, 56^3, 64^3).
 inline bool two_steps_pay(const TwoStepShape& s, uint32_t Nx, uint32_t Ny, uint32_t Nz, uint32_t q, bool trt, uint32_t ext) {
 	const uint32_t weight = ((ext & (EXT_VOLUME_FORCE | EXT_POROSITY)) ? 1u : 0u) + ((ext & EXT_POROSITY) ? 1u : 0u) + ((ext & EXT_SUBGRID) ? 2u : 0u) + (trt ? 1u : 0u) + (q == 27u ? 1u : 0u);
-	if(Ny < 2u || Nz < 4u || (uint64_t)Nx * Ny * Nz <= 65536ull << weight) return false;
+	const uint64_t ddf_bytes = (uint64_t)Nx * Ny * Nz * q * 4u;
+	if(Ny < 2u || Nz < 4u || ddf_bytes <= L2_BYTES) return false;
 	const uint64_t lanes = (uint64_t)s.tiles_x * (s.wide ? TWO_STEP_WIDE_X : TWO_STEP_NARROW_X), percent = Nx * 100ull / lanes;
+	if(ddf_bytes <= CACHED_BYTES) return weight <= 2u && percent >= (weight == 2u || 2u * ddf_bytes > CACHED_BYTES ? 85u : 75u);
 	return percent >= (weight > 2u ? 90u : s.wide ? 55u : 40u);
 }
 
@@ -354,6 +388,13 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		LbmArgs b = a;
 		b.xchunks = s.xchunks;
 		b.reverse = s.alternate ? a.odd : 0u;
+		if(s.cached) {
+			if constexpr(cached_pairs) {
+				if(s.pairs) { k_stream_collide_pair<Q, ST, TRT, EXT, pair_buffer || !pairs, true><<<s.grid, s.block, 0, st>>>(b); return; }
+			}
+			k_stream_collide<Q, ST, TRT, EXT, true, true, false, linear_buffer, true><<<s.grid, s.block, 0, st>>>(b);
+			return;
+		}
 		if(s.lin) {
 			if constexpr(linear_buffer) {
 				if(s.buf) { k_stream_collide<Q, ST, TRT, EXT, linear_xcd, true, false, true><<<s.grid, s.block, s.lds, st>>>(b); return; }
@@ -381,6 +422,7 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 	static void update_fields(const LbmArgs& a, const LaunchShape& s, hipStream_t st) {
 		LbmArgs b = a;
 		b.xchunks = s.xchunks;
+		if(s.cached) { k_update_fields<Q, ST, EXT, true, true, linear_buffer, true><<<s.grid, s.block, 0, st>>>(b); return; }
 		if(s.lin) {
 			if constexpr(linear_buffer) {
 				if(s.buf) { k_update_fields<Q, ST, EXT, linear_xcd, true, true><<<s.grid, s.block, 0, st>>>(b); return; }
@@ -402,7 +444,8 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		LbmArgs b = a;
 		b.xchunks = s.xchunks;
 		b.reverse = s.alternate ? a.odd : 0u;
-		if(s.lin) k_stream_collide_record<Q, ST, TRT, EXT, false, true><<<s.grid, s.block, 0, st>>>(b, m);
+		if(s.cached) k_stream_collide_record<Q, ST, TRT, EXT, true, true, true><<<s.grid, s.block, 0, st>>>(b, m);
+		else if(s.lin) k_stream_collide_record<Q, ST, TRT, EXT, false, true><<<s.grid, s.block, 0, st>>>(b, m);
 		else k_stream_collide_record<Q, ST, TRT, EXT, true, false><<<s.grid, s.block, 0, st>>>(b, m);
 	}
 	static void adjoint_step(const AdjointArgs& g, const LaunchShape& s, hipStream_t st) {
@@ -419,8 +462,11 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 	static void two_steps(const LbmArgs& a, void* dst, const TwoStepShape& s, hipStream_t st) {
 		if constexpr(two_step) {
 			const TwoStepArgs g = {a, dst, s.tiles_x, s.tiles_y, s.tiles, s.width, s.height, s.zlen};
-			if(s.wide) k_two_steps<Q, TRT, EXT, TWO_STEP_WIDE_X, TWO_STEP_WIDE_Y><<<s.grid, two_step_threads(TWO_STEP_WIDE_X, s.height), 0, st>>>(g);
-			else k_two_steps<Q, TRT, EXT, TWO_STEP_NARROW_X, TWO_STEP_NARROW_Y><<<s.grid, two_step_threads(TWO_STEP_NARROW_X, s.height), 0, st>>>(g);
+			const unsigned threads = two_step_threads(s.wide ? TWO_STEP_WIDE_X : TWO_STEP_NARROW_X, s.height);
+			if(s.wide && s.cached) k_two_steps<Q, TRT, EXT, TWO_STEP_WIDE_X, TWO_STEP_WIDE_Y, true><<<s.grid, threads, 0, st>>>(g);
+			else if(s.wide) k_two_steps<Q, TRT, EXT, TWO_STEP_WIDE_X, TWO_STEP_WIDE_Y, false><<<s.grid, threads, 0, st>>>(g);
+			else if(s.cached) k_two_steps<Q, TRT, EXT, TWO_STEP_NARROW_X, TWO_STEP_NARROW_Y, true><<<s.grid, threads, 0, st>>>(g);
+			else k_two_steps<Q, TRT, EXT, TWO_STEP_NARROW_X, TWO_STEP_NARROW_Y, false><<<s.grid, threads, 0, st>>>(g);
 		}
 	}
 	// Launch tuning of stream_collide: residency cap in waves per SIMD (0 = none) and grid.
@@ -428,6 +474,7 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 	static constexpr bool xcd_map = tune_xcd_map(Q, ST, EXT);
 	static constexpr bool linear_xcd = tune_linear_xcd(Q, ST, EXT);
 	static constexpr bool pairs = tune_pairs(Q, ST, TRT, EXT);
+	static constexpr bool cached_pairs = tune_cached_pairs(Q, ST, TRT, EXT);
 	static constexpr bool offsets32 = tune_offsets32(Q, ST, TRT, EXT);
 	static constexpr bool buffer = tune_buffer(Q, ST, TRT, EXT);
 	static constexpr bool pair_buffer = tune_pair_buffer(Q, ST, TRT, EXT);
@@ -449,7 +496,7 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 		static const LbmKernels k = {initialize, stream_collide, update_fields, update_force_field, mass_partial, waves_cap,
 		                             stream_collide_record, adjoint_step, objective_partial, xcd_map, transfer_fi,
 		                             update_moving_boundaries, tune_linear_large(Q, ST, EXT), linear_xcd, pairs, offsets32, buffer, pair_buffer,
-	                             linear_buffer, two_step ? two_steps : nullptr};
+	                             linear_buffer, two_step ? two_steps : nullptr, cached_pairs};
 		return &k;
 	}
 };

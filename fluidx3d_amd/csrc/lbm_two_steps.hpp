@@ -70,7 +70,7 @@ template<int Q> constexpr int plane_slot(int i, int cz) {
 // the extended tile, and one for the border columns.
 constexpr uint32_t two_step_threads(uint32_t TX, uint32_t height) { return (height + 2u) * TX + 64u; }
 
-template<int Q, bool TRT, uint32_t EXT, int TX, int TY>
+template<int Q, bool TRT, uint32_t EXT, int TX, int TY, bool CACHED>
 __global__ __launch_bounds__((two_step_threads(TX, TY))) void k_two_steps(TwoStepArgs g) {
 	constexpr int ROWS = TY + 2, PITCH = TX + 2, CELLS = ROWS * PITCH;
 	constexpr int NM = plane_slot<Q>(Q, -1), N0 = plane_slot<Q>(Q, 0), NP = plane_slot<Q>(Q, 1);
@@ -113,6 +113,10 @@ __global__ __launch_bounds__((two_step_threads(TX, TY))) void k_two_steps(TwoSte
 		slot[i + 1] = (uint64_t)(a.odd ? i + 1 : i) * a.N * 4u;
 	});
 	typedef __attribute__((address_space(1))) float gfloat;
+	const auto put = [](auto* p, float v) __attribute__((always_inline)) {
+		if constexpr(CACHED) *p = v;
+		else __builtin_nontemporal_store(v, p);
+	};
 	const auto at = [](const void* p, uint64_t uniform_bytes, uint32_t cell) __attribute__((always_inline)) {
 		return (gfloat*)((__attribute__((address_space(1))) char*)((uint64_t)p + uniform_bytes) + cell * 4u);
 	};
@@ -224,11 +228,11 @@ __global__ __launch_bounds__((two_step_threads(TX, TY))) void k_two_steps(TwoSte
 		fl1 = flk;
 		// store_f at the parity of step t+1
 		const Offsets o = offsets(z);
-		__builtin_nontemporal_store(out[0], at(g.dst, o.z[1], col));
+		put(at(g.dst, o.z[1], col), out[0]);
 		static_for<1, Q, 2>([&](auto c) __attribute__((always_inline)) {
 			constexpr int i = decltype(c)::value;
 			*at(g.dst, slot[i] + o.z[VS<Q>::cz[i] + 1], ys[VS<Q>::cy[i] + 1] + xs[VS<Q>::cx[i] + 1]) = out[i];
-			__builtin_nontemporal_store(out[i + 1], at(g.dst, slot[i + 1] + o.z[1], col));
+			put(at(g.dst, slot[i + 1] + o.z[1], col), out[i + 1]);
 		});
 	}
 }

@@ -47,11 +47,14 @@ int main() {
   auto pay = [](unsigned nx, unsigned ny, unsigned nz, unsigned q, bool trt, unsigned ext) {
     return (int)two_steps_pay(two_step_shape(nx, ny, nz, 256), nx, ny, nz, q, trt, ext);
   };
-  printf("pay %d%d%d%d%d%d%d%d%d%d%d%d%d\n", pay(256, 256, 256, 19, false, 0), pay(40, 40, 40, 19, false, 0), pay(48, 48, 48, 19, false, 0),
-         pay(130, 130, 130, 19, false, 0), pay(16, 1024, 64, 19, false, 0), pay(400, 400, 3, 19, false, 0), pay(400, 1, 400, 19, false, 0),
-         pay(64, 64, 64, 27, false, EXT_VOLUME_FORCE), pay(200, 200, 200, 27, true, EXT_VOLUME_FORCE),
-         pay(256, 256, 256, 27, true, EXT_VOLUME_FORCE), pay(128, 128, 128, 27, true, EXT_VOLUME_FORCE | EXT_POROSITY),
-         pay(200, 200, 200, 19, true, EXT_VOLUME_FORCE), pay(512, 512, 512, 19, true, EXT_EQUILIBRIUM_BOUNDARIES));
+  printf("pay %d%d%d%d%d%d%d%d%d%d%d%d%d%d%d%d\n",
+         pay(256, 256, 256, 19, false, 0), pay(64, 64, 64, 19, false, 0), pay(128, 64, 64, 19, false, 0), // L2_BYTES
+         pay(80, 80, 80, 19, false, 0), pay(96, 96, 96, 19, false, 0), pay(96, 96, 96, 19, true, EXT_VOLUME_FORCE),
+         pay(128, 128, 128, 19, true, EXT_VOLUME_FORCE), pay(128, 128, 128, 19, true, EXT_VOLUME_FORCE | EXT_POROSITY),
+         pay(201, 75, 120, 19, false, 0), pay(201, 75, 99, 19, false, 0), // both arrays in the cache or not
+         pay(130, 170, 170, 19, false, 0), pay(160, 160, 160, 19, false, 0), // above CACHED_BYTES
+         pay(16, 1024, 250, 19, false, 0), pay(2000, 2000, 3, 19, false, 0), pay(2000, 1, 2000, 19, false, 0),
+         pay(200, 200, 200, 27, true, EXT_VOLUME_FORCE));
   for (int q : {19, 27}) for (unsigned st : {ST_FP32, ST_FP16S, ST_FP16C}) for (unsigned ext : {0u, (unsigned)EXT_FORCE_FIELD, (unsigned)EXT_POROSITY, (unsigned)EXT_UPDATE_FIELDS, (unsigned)EXT_MOVING_BOUNDARIES, (unsigned)EXT_SUBGRID}) {
     const bool k = q == 19 ? tune_two_steps(19, st, true, ext ? EXT_ALL : 0u) : tune_two_steps(27, st, false, ext ? EXT_ALL : 0u);
     if (k != (st == ST_FP32 && ext == 0u)) printf("tune %d %u %u\n", q, st, ext);
@@ -77,36 +80,39 @@ def test_shapes_cover_every_cell_once(lines):
 
 
 def test_rule(lines):
-    assert lines[1:] == ["pay 1010000001111"], lines
+    assert lines[1:] == ["pay 1010101001010000"], lines
 
 
 POROUS = ("VOLUME_FORCE", "POROSITY", "PRECISE_DENSITY")
 EQ_FF = ("EQUILIBRIUM_BOUNDARIES", "FORCE_FIELD")
 # (size, q, collision, extensions): every kernel, on lattices that the rule takes
 CASES = [
-    ((128, 21, 27), 19, "SRT", ()),              # one tile across, 5-row tiles clipped to 1
-    ((64, 43, 29), 19, "SRT", ()),               # 64-wide tiles
-    ((33, 71, 31), 19, "SRT", ()),               # 31 lanes idle
-    ((257, 18, 17), 19, "SRT", ()),              # three tiles across, the last of 65 cells
-    ((300, 2, 120), 19, "SRT", ()),              # rows 0 and 1 are each other's neighbours twice
-    ((300, 60, 4), 19, "SRT", ()),
-    ((128, 64, 17), 19, "TRT", ()),
-    ((129, 64, 40), 27, "SRT", ()),              # 51 % of the lanes: single steps
-    ((160, 50, 37), 27, "TRT", ()),
-    ((160, 41, 23), 19, "SRT", EQ_FF),
-    ((100, 53, 31), 19, "TRT", ("EQUILIBRIUM_BOUNDARIES",)),
-    ((128, 64, 35), 27, "TRT", EQ_FF),
-    ((201, 33, 29), 19, "SRT", ("VOLUME_FORCE",)),
-    ((150, 61, 37), 19, "TRT", ("VOLUME_FORCE",)),
-    ((125, 91, 97), 27, "TRT", ("VOLUME_FORCE",)),
-    ((125, 91, 25), 19, "SRT", POROUS),
-    ((123, 91, 53), 19, "TRT", POROUS),
-    ((254, 71, 61), 27, "TRT", POROUS),
-    ((160, 70, 33), 19, "SRT", ("SUBGRID",)),
-    ((128, 70, 61), 19, "TRT", ("EQUILIBRIUM_BOUNDARIES", "SUBGRID")),
-    ((150, 40, 33), 19, "SRT", ("MOVING_BOUNDARIES",)),
-    ((100, 63, 47), 27, "SRT", ("MOVING_BOUNDARIES", "FORCE_FIELD", "EQUILIBRIUM_BOUNDARIES")),
-    ((128, 91, 97), 27, "TRT", ("MOVING_BOUNDARIES", "SUBGRID")),
+    ((128, 61, 58), 19, "SRT", ()),              # one tile across, clipped in y and z
+    ((64, 143, 51), 19, "SRT", ()),              # 64-wide tiles
+    ((50, 143, 63), 19, "SRT", ()),              # 14 lanes idle
+    ((257, 81, 34), 19, "SRT", ()),              # three tiles across, the last of 65 cells
+    ((350, 81, 82), 19, "SRT", ()),              # 91 %, one array of two in the caches
+    ((300, 2, 800), 19, "SRT", ()),              # rows 0 and 1 are each other's neighbours twice
+    ((300, 400, 4), 19, "SRT", ()),
+    ((128, 64, 61), 19, "TRT", ()),
+    ((257, 151, 84), 19, "SRT", ()),             # above CACHED_BYTES, 66 %
+    ((129, 64, 60), 27, "SRT", ()),              # 51 % of the lanes: single steps
+    ((250, 50, 37), 27, "TRT", ()),
+    ((240, 41, 53), 19, "SRT", EQ_FF),
+    ((100, 73, 61), 19, "TRT", ("EQUILIBRIUM_BOUNDARIES",)),
+    ((128, 64, 45), 27, "TRT", EQ_FF),
+    ((251, 53, 39), 19, "SRT", ("VOLUME_FORCE",)),
+    ((120, 91, 47), 19, "TRT", ("VOLUME_FORCE",)),
+    ((125, 191, 97), 27, "TRT", ("VOLUME_FORCE",)),   # above CACHED_BYTES from here
+    ((125, 191, 131), 19, "SRT", POROUS),
+    ((123, 191, 133), 19, "TRT", POROUS),
+    ((254, 71, 131), 27, "TRT", POROUS),
+    ((160, 170, 133), 19, "SRT", ("SUBGRID",)),
+    ((128, 70, 61), 19, "SRT", ("EQUILIBRIUM_BOUNDARIES", "SUBGRID")),
+    ((128, 140, 173), 19, "TRT", ("EQUILIBRIUM_BOUNDARIES", "SUBGRID")),
+    ((240, 40, 53), 19, "SRT", ("MOVING_BOUNDARIES",)),
+    ((100, 63, 57), 27, "SRT", ("MOVING_BOUNDARIES", "FORCE_FIELD", "EQUILIBRIUM_BOUNDARIES")),
+    ((128, 191, 97), 27, "TRT", ("MOVING_BOUNDARIES", "SUBGRID")),
 ]
 
 
@@ -151,7 +157,7 @@ def test_run_equals_single_steps(size, q, collision, extensions):
 @pytest.mark.gpu
 def test_run_equals_oracle(oracle):
     import fluidx3d_amd as fx
-    size = (150, 41, 13)
+    size = (128, 64, 55)
     lbm = scene_lbm(fx, size, 19, "TRT", ())
     rho, u, flags = scenes.random_scene(*size, seed=5)
     ref = oracle.OracleLBM(*size, w=lbm.w, trt=True)
@@ -171,10 +177,10 @@ def test_adjoint_forward_equals_single_steps():
     between checkpoints taken two steps at a time."""
     import fluidx3d_amd as fx
     from fluidx3d_amd.adjoint import Adjoint
-    rho, u, flags, alpha = scenes.porous_channel(128, 40, 52)
+    rho, u, flags, alpha = scenes.porous_channel(128, 64, 58)
     states = []
     for interval in (9, 1):  # an interval of 1 leaves single steps only
-        lbm = fx.LBM(128, 40, 52, 1.0 / 6.0, 1e-5, 0.0, 0.0, extensions=POROUS)
+        lbm = fx.LBM(128, 64, 58, 1.0 / 6.0, 1e-5, 0.0, 0.0, extensions=POROUS)
         lbm.rho.host[:], lbm.u.host[:], lbm.flags.host[:], lbm.porosity.host[:] = rho, u, flags, alpha
         adj = Adjoint(lbm, steps=31, window_begin=25, plane_x=127, checkpoint_interval=interval)
         states.append((adj.forward(), lbm.read_ddfs(), adj.backward()))
