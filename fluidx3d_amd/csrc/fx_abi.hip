@@ -64,7 +64,6 @@ struct fx_adjoint {
 	void* work_fi = nullptr;    // recomputation state
 	float* moments = nullptr;   // k * 4 * N
 	float* lambda = nullptr;    // q * N
-	double* partial = nullptr;  // obj_blocks
 	double* acc = nullptr;      // 1
 	bool forward_done = false;
 };
@@ -173,7 +172,8 @@ int ensure_partial(fx_ctx* ctx, uint64_t doubles) {
 struct SecondArray {
 	fx_ctx* ctx;
 	void* array = nullptr;
-	explicit SecondArray(fx_ctx* c) : ctx(c) {
+	explicit SecondArray(fx_ctx* c, bool wanted = true) : ctx(c) {
+		if(!wanted) return;
 		std::lock_guard<std::mutex> lock(g_second_mutex);
 		if(ctx->second_busy) return; // another thread is queueing launches on it
 		if(!ctx->second) {
@@ -390,6 +390,31 @@ __global__ __launch_bounds__(RED_BLOCK) void k_reduce_add(const double* partial,
 		__syncthreads();
 	}
 	if(threadIdx.x == 0) acc[0] += red[0];
+}
+
+// totals[b]: the sum that k_reduce_add forms of the `count` partials of step b.
+__global__ __launch_bounds__(RED_BLOCK) void k_reduce_each(const double* partial, uint64_t count, double* totals) {
+	__shared__ double red[RED_BLOCK];
+	partial += blockIdx.x * count;
+	double s = 0.0;
+	for(uint64_t b = threadIdx.x; b < count; b += RED_BLOCK) s += partial[b];
+	red[threadIdx.x] = s;
+	__syncthreads();
+	for(int h = RED_BLOCK / 2; h > 0; h >>= 1) {
+		if((int)threadIdx.x < h) red[threadIdx.x] += red[threadIdx.x + h];
+		__syncthreads();
+	}
+	if(threadIdx.x == 0) totals[blockIdx.x] = red[0];
+}
+// acc += totals[0], then totals[1], ...: one wave.
+__global__ __launch_bounds__(64) void k_add_in_order(const double* totals, uint64_t count, double* acc) {
+	double s = acc[0];
+	for(uint64_t b = 0; b < count; b += 64u) {
+		const double v = b + threadIdx.x < count ? totals[b + threadIdx.x] : 0.0;
+		const int n = count - b < 64u ? (int)(count - b) : 64;
+		for(int i = 0; i < n; i++) s += __shfl(v, i);
+	}
+	if(threadIdx.x == 0) acc[0] = s;
 }
 
 // Element-wise kernels run a grid-stride loop over a grid of at most STRIDE_BLOCKS blocks,
@@ -610,6 +635,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 			ctx->shape_sc.cached = true;
 		} else ctx->shape_sc = fx::slab_shape(N);
 		ctx->shape_rec = fx::slab_shape(N);
+		if(N * cfg->velocity_set * 8u <= fx::CACHED_BYTES) ctx->shape_adj = fx::slab_shape(N);
 		if(ddf + 17u * N <= fx::CACHED_BYTES) ctx->shape_uf = fx::slab_shape(N); // the DDFs and what update_fields writes
 	}
 	ctx->shape_sc.alternate = N * cfg->velocity_set * eb >= fx::ALTERNATE_ORDER_BYTES;
@@ -891,8 +917,7 @@ static int adjoint_layout(const fx_ctx* ctx, const fx_adjoint_config* cfg, uint6
 	if(k > cfg->steps) k = cfg->steps;
 	checkpoints = (cfg->steps + k - 1u) / k;
 	const uint64_t N = ctx->N, q = ctx->cfg.velocity_set;
-	const uint64_t obj_blocks = ((uint64_t)ctx->cfg.Ny * ctx->cfg.Nz + 255u) / 256u;
-	bytes = checkpoints * ddf_bytes(ctx) + ddf_bytes(ctx) + k * 4u * N * 4u + q * N * 4u + (obj_blocks + 1u) * 8u;
+	bytes = checkpoints * ddf_bytes(ctx) + ddf_bytes(ctx) + k * 4u * N * 4u + q * N * 4u + 8u;
 	return FX_OK;
 }
 
@@ -922,7 +947,6 @@ int fx_adjoint_create(fx_ctx* ctx, const fx_adjoint_config* cfg, fx_adjoint** ou
 	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->work_fi, adj->fi_bytes);
 	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->moments, k * 4u * ctx->N * sizeof(float));
 	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->lambda, (uint64_t)ctx->cfg.velocity_set * ctx->N * sizeof(float));
-	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->partial, adj->obj_blocks * sizeof(double));
 	if(e == hipSuccess) e = allocate_device(ctx->device, (void**)&adj->acc, sizeof(double));
 	if(e != hipSuccess) { fx_adjoint_destroy(adj); return fail(FX_ERR_MEMORY, std::string("adjoint workspace: ") + hipGetErrorString(e)); }
 	*out = adj;
@@ -937,7 +961,6 @@ int fx_adjoint_destroy(fx_adjoint* adj) {
 	if(adj->work_fi) (void)hipFree(adj->work_fi);
 	if(adj->moments) (void)hipFree(adj->moments);
 	if(adj->lambda) (void)hipFree(adj->lambda);
-	if(adj->partial) (void)hipFree(adj->partial);
 	if(adj->acc) (void)hipFree(adj->acc);
 	delete adj;
 	return FX_OK;
@@ -951,7 +974,7 @@ int fx_lbm_stream_collide_record(fx_ctx* ctx, void* fi, float* rho, float* u, co
 	if(ctx->cfg.extensions & (FX_MOVING_BOUNDARIES | FX_SUBGRID))
 		return fail(FX_ERR_CONFIG, "the adjoint does not differentiate MOVING_BOUNDARIES or SUBGRID");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	ctx->k->stream_collide_record(make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), ctx->shape_rec, ctx->stream, moments);
+	ctx->k->stream_collide_record(make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), ctx->shape_rec, ctx->stream, moments, fi);
 	return check_launch("stream_collide_record");
 }
 
@@ -980,12 +1003,6 @@ int fx_lbm_adjoint_step(fx_ctx* ctx, float* lambda, const float* rho, const floa
 	return check_launch("adjoint_step");
 }
 
-static int objective_accumulate(fx_ctx* ctx, const void* fi, const uint8_t* flags, uint64_t t, uint32_t plane_x, double* partial, uint64_t blocks, double* acc) {
-	ctx->k->objective_partial(make_args(ctx, fi, nullptr, nullptr, flags, t, 0.0f, 0.0f, 0.0f, nullptr, nullptr), plane_x, ctx->stream, partial);
-	fx::k_reduce_add<<<1, fx::RED_BLOCK, 0, ctx->stream>>>(partial, blocks, acc);
-	return check_launch("objective");
-}
-
 int fx_lbm_objective_plane(fx_ctx* ctx, const void* fi, const uint8_t* flags, uint64_t t, uint32_t plane_x, double* out) {
 	if(!ctx || !fi || !flags || !out) return fail(FX_ERR_ARG, "null argument");
 	if(plane_x >= ctx->cfg.Nx) return fail(FX_ERR_ARG, "plane_x out of range");
@@ -994,7 +1011,9 @@ int fx_lbm_objective_plane(fx_ctx* ctx, const void* fi, const uint8_t* flags, ui
 	int rc = ensure_partial(ctx, blocks);
 	if(rc != FX_OK) return rc;
 	FX_HIP(hipMemsetAsync(ctx->result, 0, sizeof(double), ctx->stream));
-	rc = objective_accumulate(ctx, fi, flags, t, plane_x, ctx->partial, blocks, ctx->result);
+	ctx->k->objective_partial(make_args(ctx, fi, nullptr, nullptr, flags, t, 0.0f, 0.0f, 0.0f, nullptr, nullptr), plane_x, ctx->stream, ctx->partial);
+	fx::k_reduce_add<<<1, fx::RED_BLOCK, 0, ctx->stream>>>(ctx->partial, blocks, ctx->result);
+	rc = check_launch("objective");
 	if(rc != FX_OK) return rc;
 	FX_HIP(hipMemcpyAsync(out, ctx->result, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
 	FX_HIP(hipStreamSynchronize(ctx->stream));
@@ -1010,18 +1029,55 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 	const fx_adjoint_config& c = adj->cfg;
 	FX_HIP(hipMemsetAsync(adj->acc, 0, sizeof(double), ctx->stream));
 	FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-	const fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, 0u, fx_, fy_, fz_, F, alpha);
+	fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, 0u, fx_, fy_, fz_, F, alpha);
+	// The objective's partial sums of each step and their totals lie in lambda, which only the
+	// backward sweep uses; they are added in the order of the steps.
+	double* const partial = (double*)adj->lambda;
+	const uint64_t batch = std::min<uint64_t>((uint64_t)ctx->cfg.velocity_set * ctx->N / 2u / (adj->obj_blocks + 1u), 1u << 16);
+	uint64_t summed = 0;
+	const auto sum_objective = [&]() {
+		double* const totals = partial + summed * adj->obj_blocks;
+		fx::k_reduce_each<<<(unsigned)summed, fx::RED_BLOCK, 0, ctx->stream>>>(partial, adj->obj_blocks, totals);
+		fx::k_add_in_order<<<1, 64, 0, ctx->stream>>>(totals, summed, adj->acc);
+		summed = 0;
+	};
+	// Before the window every span of steps runs from one checkpoint to the next or to the
+	// window: pairs of steps from the checkpoint, fi and the second array in turn, to the next
+	// checkpoint, so that no copy of the DDFs is made.
+	const SecondArray second(ctx, ctx->shape_two.grid && adj->k >= 2u && c.window_begin >= 2u);
+	void* now = fi; // the state of step t
 	for(uint64_t t = 0, n = 0; t < c.steps; t += n) {
-		if(t % adj->k == 0u) FX_HIP(hipMemcpyAsync(adj->ckpt + (t / adj->k) * adj->fi_bytes, fi, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
+		void* const saved = adj->ckpt + (t / adj->k) * adj->fi_bytes;
+		if(t % adj->k == 0u && now != saved) FX_HIP(hipMemcpyAsync(saved, now, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
 		if(t >= c.window_begin) {
-			rc = objective_accumulate(ctx, fi, flags, t, c.plane_x, adj->partial, adj->obj_blocks, adj->acc);
-			if(rc != FX_OK) return rc;
+			if(now != fi) FX_HIP(hipMemcpyAsync(fi, now, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
+			now = fi;
+			a.odd = (uint32_t)(t & 1u);
+			ctx->k->objective_partial(a, c.plane_x, ctx->stream, partial + summed * adj->obj_blocks);
+			if(++summed == batch) sum_objective();
+			queue_steps(ctx, a, t, 1u);
 			n = 1u; // the objective looks at every step
-		} else {
-			n = std::min(adj->k - t % adj->k, c.window_begin - t); // up to the next checkpoint or the window (window_begin < steps)
+			continue;
 		}
-		queue_steps(ctx, a, t, n);
+		n = std::min(adj->k - t % adj->k, c.window_begin - t); // up to the next checkpoint or the window (window_begin < steps)
+		const uint64_t pairs = second.array ? n / 2u : 0u;
+		fx::LbmArgs b = a;
+		b.odd = (uint32_t)(t & 1u);
+		if(pairs > 0u) {
+			b.fi = saved;
+			void* const end = n % 2u == 0u && (t + n) % adj->k == 0u ? (char*)saved + adj->fi_bytes : fi;
+			for(uint64_t left = pairs; left-- > 0u;) {
+				now = left == 0u ? end : (left & 1u) ? second.array : fi;
+				ctx->k->two_steps(b, now, ctx->shape_two, ctx->stream);
+				b.fi = now;
+			}
+		} else if(now != fi) {
+			FX_HIP(hipMemcpyAsync(fi, now, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
+			now = fi;
+		}
+		queue_steps(ctx, a, t + 2u * pairs, n - 2u * pairs);
 	}
+	if(summed > 0u) sum_objective();
 	rc = check_launch("forward");
 	if(rc != FX_OK) return rc;
 	FX_HIP(hipEventRecord(ctx->ev1, ctx->stream));
@@ -1055,10 +1111,10 @@ int fx_lbm_backward(fx_ctx* ctx, fx_adjoint* adj, const float* rho, const float*
 	a.ext &= ~FX_UPDATE_FIELDS; // the recomputation must not overwrite rho/u
 	for(uint64_t s = adj->checkpoints; s-- > 0u;) {
 		const uint64_t ts = s * adj->k, te = std::min<uint64_t>(c.steps, ts + adj->k);
-		FX_HIP(hipMemcpyAsync(adj->work_fi, adj->ckpt + s * adj->fi_bytes, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
-		for(uint64_t t = ts; t < te; t++) {
+		for(uint64_t t = ts; t < te; t++) { // the first step from the checkpoint, which stays
+			a.fi = t == ts ? (void*)(adj->ckpt + s * adj->fi_bytes) : adj->work_fi;
 			a.odd = (uint32_t)(t & 1u);
-			ctx->k->stream_collide_record(a, ctx->shape_rec, ctx->stream, adj->moments + (t - ts) * 4u * N);
+			ctx->k->stream_collide_record(a, ctx->shape_rec, ctx->stream, adj->moments + (t - ts) * 4u * N, adj->work_fi);
 		}
 		for(uint64_t t = te; t-- > ts;) {
 			fx::AdjointArgs g = adjoint_args(ctx, adj->lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, adj->moments + (t - ts) * 4u * N,

@@ -1015,7 +1015,7 @@ template<bool XCD, bool LIN, bool CACHED = false> __device__ __forceinline__ boo
 }
 // One lane per cell.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool RECORD, bool XCD, bool LIN, bool O32 = false, bool BUF = false, bool CACHED = false>
-__device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments) {
+__device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments, void* dst) {
 	a.ext &= EXT;
 	if constexpr(constant_vf_mask<TRT>(Q, ST, EXT, LIN)) a.ext = EXT_VOLUME_FORCE;
 	uint32_t x, y, z;
@@ -1025,9 +1025,22 @@ __device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments) {
 	const uint64_t n = s.n();
 	const uint32_t flagsn = a.flags[n];
 	const uint32_t bo = flagsn & TYPE_BO;
-	if(bo == TYPE_S || (flagsn & TYPE_SU) == TYPE_G) return; // solid cells are mailboxes
 	typedef typename Storage<ST>::E E;
 	E* fi = (E*)a.fi;
+	if(bo == TYPE_S || (flagsn & TYPE_SU) == TYPE_G) { // solid cells are mailboxes
+		if constexpr(RECORD) {
+			if(dst != a.fi) { // what they hold for the next step
+				((E*)dst)[n] = fi[n];
+#pragma unroll
+				for(int i = 1; i < Q; i += 2) {
+					const uint64_t own = (uint64_t)(a.odd ? i : i + 1) * a.N + n, shifted = (uint64_t)(a.odd ? i + 1 : i) * a.N + neighbour<Q>(s, i);
+					((E*)dst)[own] = fi[own];
+					((E*)dst)[shifted] = fi[shifted];
+				}
+			}
+		}
+		return;
+	}
 	float f[Q];
 	if constexpr(ST == ST_FP16S) {
 		// every load is issued before the first decode: left alone, the scheduler may
@@ -1044,14 +1057,14 @@ __device__ __forceinline__ void stream_collide_cell(LbmArgs a, float* moments) {
 	}
 	if((a.ext & EXT_MOVING_BOUNDARIES) && bo == TYPE_MS) moving_boundaries<Q>(a, s, f);
 	collide_cell<Q, TRT, EXT, RECORD, shared_division(ST, EXT), shared_pair_difference(Q, EXT, BUF)>(a, n, bo, f, moments);
-	store_f<Q, ST, U, LIN, O32, BUF, CACHED>(fi, a.N, s, a.odd, f);
+	store_f<Q, ST, U, LIN, O32, BUF, CACHED>((E*)dst, a.N, s, a.odd, f);
 }
 // XCD: the kernel may run on the 1-D XCD-mapped grid (a.xchunks > 0); false compiles the
 // mapping out.  LIN: the cell-linear grid (cell_coords), for lattices whose rows do not
 // start on 128-byte lines.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false, bool O32 = false, bool BUF = false, bool CACHED = false>
 __global__ __launch_bounds__(BLOCK) void k_stream_collide(LbmArgs a) {
-	stream_collide_cell<Q, ST, TRT, EXT, false, XCD, LIN, O32, BUF, CACHED>(a, nullptr);
+	stream_collide_cell<Q, ST, TRT, EXT, false, XCD, LIN, O32, BUF, CACHED>(a, nullptr, a.fi);
 }
 // stream_collide with two adjacent cells per lane, for the 16-bit formats on rows of whole
 // waves of lanes (Nx a multiple of 128, pair_rows).  A wave takes the 128 cells c0 .. c0+127
@@ -1223,10 +1236,10 @@ __global__ __launch_bounds__(BLOCK) void k_stream_collide_pair(LbmArgs a) {
 // stream_collide that also writes the pre-collision (rho, jx, jy, jz) of every fluid cell to
 // moments[c*N+n], c = 0..3 (16 B/cell): what the adjoint step needs of the forward state.
 // EXT is the context's extension subset; MOVING_BOUNDARIES and SUBGRID are not
-// differentiated and compiled out.
+// differentiated and compiled out.  dst: a.fi, or another array that then holds the next state.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT, bool XCD = false, bool LIN = false, bool CACHED = false>
-__global__ __launch_bounds__(BLOCK) void k_stream_collide_record(LbmArgs a, float* moments) {
-	stream_collide_cell<Q, ST, TRT, EXT & ~(EXT_MOVING_BOUNDARIES | EXT_SUBGRID), true, XCD, LIN, false, false, CACHED>(a, moments);
+__global__ __launch_bounds__(BLOCK) void k_stream_collide_record(LbmArgs a, float* moments, void* dst) {
+	stream_collide_cell<Q, ST, TRT, EXT & ~(EXT_MOVING_BOUNDARIES | EXT_SUBGRID), true, XCD, LIN, false, false, CACHED>(a, moments, dst);
 }
 
 // update_fields (src/kernel.cpp:1794-1870), on the grids of stream_collide (cell_coords).
@@ -1430,11 +1443,15 @@ struct AdjointArgs {
 	float obj_weight;        // objective weight of step t (0 outside the averaging window)
 };
 
-template<int Q, bool TRT, bool XCD = false, bool LIN = false>
+// SLAB: the slabs of slab_segment, where the states of the adjoint and of the recomputation stay
+// in the last-level cache (2 q N floats up to CACHED_BYTES): record pass and adjoint step, us, 64^3 21.4 -> 19.8,
+// 128x64x64 39.2 -> 38.4, 96^3 TRT 64.4 -> 61.7; 150x150x130 220 -> 223, 128^3 D3Q27 SRT FP16C 152 -> 157.
+// Non-temporal throughout: cached accesses 128^3 +3 to +5 %, 160^3 +7 %.
+template<int Q, bool TRT, bool XCD = false, bool LIN = false, bool SLAB = false>
 __global__ __launch_bounds__(BLOCK) void k_adjoint_step(AdjointArgs g) {
 	const LbmArgs& a = g.a;
 	uint32_t x, y, z;
-	if(!cell_coords<XCD, LIN>(a, x, y, z)) return;
+	if(!cell_coords<XCD, LIN, SLAB>(a, x, y, z)) return;
 	const Site s = make_site(x, y, z, a.Nx, a.Ny, a.Nz);
 	const uint64_t n = s.n();
 	const uint32_t flagsn = a.flags[n];
@@ -1579,7 +1596,7 @@ __global__ __launch_bounds__(256) void k_objective_partial(LbmArgs a, uint32_t p
 	const uint64_t m = (uint64_t)blockIdx.x * 256u + threadIdx.x;
 	double v = 0.0;
 	if(m < (uint64_t)a.Ny * a.Nz) {
-		const uint32_t y = (uint32_t)(m % a.Ny), z = (uint32_t)(m / a.Ny);
+		const uint32_t z = (m >> 31) == 0u ? a.by_Ny.quotient((uint32_t)m) : (uint32_t)(m / a.Ny), y = (uint32_t)(m - (uint64_t)z * a.Ny);
 		const Site s = make_site(plane_x, y, z, a.Nx, a.Ny, a.Nz);
 		if((a.flags[s.n()] & TYPE_BO) != TYPE_S) {
 			float f[Q];

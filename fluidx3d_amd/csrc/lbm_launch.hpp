@@ -159,7 +159,7 @@ inline LaunchShape adjoint_shape(uint32_t Nx, uint32_t Ny, uint32_t Nz) { return
 
 typedef void (*lattice_fn)(const LbmArgs&, const LaunchShape&, hipStream_t);
 typedef void (*mass_fn)(const LbmArgs&, const LaunchShape&, hipStream_t, double*);
-typedef void (*record_fn)(const LbmArgs&, const LaunchShape&, hipStream_t, float*);
+typedef void (*record_fn)(const LbmArgs&, const LaunchShape&, hipStream_t, float*, void* dst);
 typedef void (*two_steps_fn)(const LbmArgs&, void*, const TwoStepShape&, hipStream_t);
 typedef void (*adjoint_fn)(const AdjointArgs&, const LaunchShape&, hipStream_t);
 typedef void (*objective_fn)(const LbmArgs&, uint32_t, hipStream_t, double*);
@@ -440,19 +440,20 @@ template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {
 	static void update_moving_boundaries(const LbmArgs& a, const LaunchShape& s, hipStream_t st) { k_update_moving_boundaries<Q><<<s.grid, s.block, 0, st>>>(a); }
 	// the adjoint kernels run on the XCD-mapped grid when rows take several blocks
 	// (adjoint_shape); measured at 384x192x192: record pass +14 %, adjoint step +10 %
-	static void stream_collide_record(const LbmArgs& a, const LaunchShape& s, hipStream_t st, float* m) {
+	static void stream_collide_record(const LbmArgs& a, const LaunchShape& s, hipStream_t st, float* m, void* dst) {
 		LbmArgs b = a;
 		b.xchunks = s.xchunks;
 		b.reverse = s.alternate ? a.odd : 0u;
-		if(s.cached) k_stream_collide_record<Q, ST, TRT, EXT, true, true, true><<<s.grid, s.block, 0, st>>>(b, m);
-		else if(s.lin) k_stream_collide_record<Q, ST, TRT, EXT, false, true><<<s.grid, s.block, 0, st>>>(b, m);
-		else k_stream_collide_record<Q, ST, TRT, EXT, true, false><<<s.grid, s.block, 0, st>>>(b, m);
+		if(s.cached) k_stream_collide_record<Q, ST, TRT, EXT, true, true, true><<<s.grid, s.block, 0, st>>>(b, m, dst);
+		else if(s.lin) k_stream_collide_record<Q, ST, TRT, EXT, false, true><<<s.grid, s.block, 0, st>>>(b, m, dst);
+		else k_stream_collide_record<Q, ST, TRT, EXT, true, false><<<s.grid, s.block, 0, st>>>(b, m, dst);
 	}
 	static void adjoint_step(const AdjointArgs& g, const LaunchShape& s, hipStream_t st) {
 		AdjointArgs h = g;
 		h.a.xchunks = s.xchunks;
 		h.a.reverse = s.alternate ? g.a.odd : 0u;
-		if(s.lin) k_adjoint_step<Q, TRT, false, true><<<s.grid, s.block, 0, st>>>(h);
+		if(s.cached) k_adjoint_step<Q, TRT, true, true, true><<<s.grid, s.block, 0, st>>>(h);
+		else if(s.lin) k_adjoint_step<Q, TRT, false, true><<<s.grid, s.block, 0, st>>>(h);
 		else k_adjoint_step<Q, TRT, true, false><<<s.grid, s.block, 0, st>>>(h);
 	}
 	static void objective_partial(const LbmArgs& a, uint32_t plane_x, hipStream_t st, double* p) {

@@ -172,19 +172,21 @@ def test_run_equals_oracle(oracle):
 
 
 @pytest.mark.gpu
-def test_adjoint_forward_equals_single_steps():
-    """Adjoint.forward: the objective and the checkpointed gradient's inputs with the spans
-    between checkpoints taken two steps at a time."""
+@pytest.mark.parametrize("interval,window", [(9, 25), (10, 25), (10, 20), (10, 21), (10, 2), (4, 30), (31, 30), (5, 0)])
+def test_adjoint_equals_single_steps(interval, window):
+    """Adjoint.forward: the objective, the DDFs and the gradient with the spans between
+    checkpoints taken two steps at a time, from one checkpoint to the next (an even interval),
+    back into the lattice's own array (an odd one, the window), and spans of one step."""
     import fluidx3d_amd as fx
     from fluidx3d_amd.adjoint import Adjoint
     rho, u, flags, alpha = scenes.porous_channel(128, 64, 58)
     states = []
-    for interval in (9, 1):  # an interval of 1 leaves single steps only
+    for k in (interval, 1):  # an interval of 1 leaves single steps only
         lbm = fx.LBM(128, 64, 58, 1.0 / 6.0, 1e-5, 0.0, 0.0, extensions=POROUS)
         lbm.rho.host[:], lbm.u.host[:], lbm.flags.host[:], lbm.porosity.host[:] = rho, u, flags, alpha
-        adj = Adjoint(lbm, steps=31, window_begin=25, plane_x=127, checkpoint_interval=interval)
-        states.append((adj.forward(), lbm.read_ddfs(), adj.backward()))
+        adj = Adjoint(lbm, steps=31, window_begin=window, plane_x=127, checkpoint_interval=k)
+        states.append((adj.forward(), lbm.read_ddfs(), adj.backward(), adj.backward()))
         adj.close()
         lbm.close()
-    (J, f, g), (J1, f1, g1) = states
-    assert J == J1 and np.array_equal(f, f1) and np.array_equal(g, g1)
+    (J, f, g, again), (J1, f1, g1, _) = states
+    assert J == J1 and np.array_equal(f, f1) and np.array_equal(g, g1) and np.array_equal(g, again)
