@@ -178,10 +178,14 @@ int fx_lbm_update_moving_boundaries(fx_ctx* ctx, const float* u, uint8_t* flags)
 int fx_lbm_stream_collide(fx_ctx* ctx, void* fi, float* rho, float* u, const uint8_t* flags,
                           uint64_t t, float fx, float fy, float fz, const float* F, const float* alpha);
 
-/* steps consecutive stream_collide launches for t = t0 .. t0+steps-1, bracketed by HIP
- * events on the context stream; waits and returns the elapsed milliseconds in *ms
- * (may be NULL: then it does not wait).  Replaces the loop of LBM::run
- * (src/lbm.cpp:955-975) without the per-step host synchronisation of src/lbm.cpp:951. */
+/* The time steps t = t0 .. t0+steps-1, queued back to back on the context stream; with ms
+ * not NULL bracketed by HIP events, and the call waits and returns the elapsed milliseconds.
+ * FP32 lattices on which it is faster take two steps per launch, with a second DDF array that the
+ * context allocates once if half of the device memory stays free, keeps, and gives back when an
+ * allocation through this interface would fail without it; otherwise, and with an array that
+ * cannot be had, each step is a stream_collide launch.  The results are the same bits.
+ * Replaces the loop of LBM::run (src/lbm.cpp:955-975) without the per-step host
+ * synchronisation of src/lbm.cpp:951. */
 int fx_lbm_run(fx_ctx* ctx, void* fi, float* rho, float* u, const uint8_t* flags, uint64_t t0, uint64_t steps,
                float fx, float fy, float fz, const float* F, const float* alpha, float* ms);
 
@@ -248,7 +252,8 @@ typedef struct fx_adjoint fx_adjoint;
 int fx_adjoint_memory(const fx_ctx* ctx, const fx_adjoint_config* cfg, uint64_t* bytes);
 int fx_adjoint_create(fx_ctx* ctx, const fx_adjoint_config* cfg, fx_adjoint** out);
 int fx_adjoint_destroy(fx_adjoint* adj);
-/* forward pass with checkpoints; *objective = J; *ms = GPU time (either may be NULL) */
+/* forward pass with checkpoints; *objective = J; *ms = GPU time (either may be NULL).  Steps
+ * before the window go two per launch where fx_lbm_run's do */
 int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u, const uint8_t* flags,
                    float fx, float fy, float fz, const float* F, const float* alpha, double* objective, float* ms);
 /* checkpointed adjoint sweep after fx_lbm_forward; rho/u hold the TYPE_E presets */
