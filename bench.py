@@ -15,7 +15,7 @@ back to back on the context stream and bracketed by HIP events on that stream
 the median batch (min and max reported beside it).  roofline.achieved = the bytes that a
 launch has to move (bandwidth_bytes_per_cell_device, src/lbm.cpp:51-72: 153 B FP32, 77 B FP16
 per cell, for the two steps of an FP32 launch together) / the median batch's average launch
-duration; peak = 8000 GB/s (MI355X).
+duration, with the launches that the library counted; peak = 8000 GB/s (MI355X).
 The device copy peak is measured first.  Beside the headline: the two sphere-flow
 lattices (512x256x256 D3Q27 TRT FP16C with equilibrium boundaries and the force field,
 1536x768x768 D3Q19 SRT FP16S), the checkpointed adjoint against the plain forward step,
@@ -96,18 +96,25 @@ def sync_leg(L, ctx, args, t, steps, F=None):
     return (time.perf_counter() - t0) / max(steps, 1), t
 
 
-def rate_summary(N, bpc, batch_ms, steps, steps_per_launch=1):
+def step_launches(ctx):
+    """Launches for time steps so far; each reads and writes every DDF once, for one or two steps."""
+    n = ctx.launches()
+    return n.one_step + n.two_steps
+
+
+def rate_summary(N, bpc, batch_ms, steps, launches):
     """MLUPs/s of the median batch (min and max beside it) and its roofline figures; bpc:
-    bytes per cell and launch."""
-    per_launch = sorted(b / steps for b in batch_ms)
-    med = per_launch[len(per_launch) // 2]
+    bytes per cell and launch; launches: of all batches together."""
+    per_step = sorted(b / steps for b in batch_ms)
+    med = per_step[len(per_step) // 2]
+    steps_per_launch = steps * len(batch_ms) / launches
     gbps = bpc * N / (med * steps_per_launch * 1e-3) * 1e-9
     return {
         "mlups": N / (med * 1e-3) * 1e-6,
-        "mlups_min": N / (per_launch[-1] * 1e-3) * 1e-6,
-        "mlups_max": N / (per_launch[0] * 1e-3) * 1e-6,
+        "mlups_min": N / (per_step[-1] * 1e-3) * 1e-6,
+        "mlups_max": N / (per_step[0] * 1e-3) * 1e-6,
         "ms_per_step": med,
-        "batches": len(per_launch),
+        "batches": len(per_step),
         "bytes_per_cell": bpc,
         "steps_per_launch": steps_per_launch,
         "achieved_GBps": gbps,
@@ -132,15 +139,14 @@ def gpu_mode(fx, size, storage, steps, warmup, sync_steps, repeats):
     _, t = timed_batches(L, args, 0, warmup, 1)
     sync_s, t = sync_leg(L, lbm.ctx, args, t, sync_steps)
     lbm.ctx.sync()
+    before = step_launches(lbm.ctx)
     wall0 = time.perf_counter()
     batch_ms, t = timed_batches(L, args, t, steps, repeats)
     lbm.ctx.sync()
     wall = time.perf_counter() - wall0
     lbm.t = t
     N = lbm.N
-    # FP32 cubes of this size take two steps per launch (two_steps_pay in lbm_launch.hpp)
-    pairs = storage == "FP32" and size % 64 == 0 and size > 64
-    out = rate_summary(N, fx.bandwidth_bytes_per_cell(lbm.cfg), batch_ms, steps, 2 if pairs else 1)
+    out = rate_summary(N, fx.bandwidth_bytes_per_cell(lbm.cfg), batch_ms, steps, step_launches(lbm.ctx) - before)
     out["wall_mlups"] = N * steps * repeats / wall * 1e-6
     out["per_step_sync_mlups"] = N / sync_s * 1e-6
     out["mass_rel_drift"] = f"{abs(lbm.mass() - m0) / m0:.3e}"
@@ -197,10 +203,11 @@ def sphere_leg(fx, name, dims, radius, velocity_set, collision, storage, extensi
     F = lbm.F.device if lbm.F is not None else None
     _, t = timed_batches(L, args, 0, warmup, 1, F=F)
     sync_s, t = sync_leg(L, lbm.ctx, args, t, sync_steps, F=F)
+    before = step_launches(lbm.ctx)
     batch_ms, t = timed_batches(L, args, t, steps, repeats, F=F)
     lbm.t = t
     out = {"workload": name}
-    out.update(rate_summary(N, fx.bandwidth_bytes_per_cell(lbm.cfg), batch_ms, steps))
+    out.update(rate_summary(N, fx.bandwidth_bytes_per_cell(lbm.cfg), batch_ms, steps, step_launches(lbm.ctx) - before))
     if "FORCE_FIELD" in extensions and "VOLUME_FORCE" not in extensions:
         # the byte count above includes 12 B/cell of force field (src/lbm.cpp:60-62), but
         # without VOLUME_FORCE stream_collide never uses F, so neither kernel reads it

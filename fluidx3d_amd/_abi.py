@@ -22,6 +22,8 @@ FX_POROSITY = 16
 FX_PRECISE_DENSITY = 32
 FX_MOVING_BOUNDARIES = 64
 FX_SUBGRID = 128
+FX_FORM_TWO_STEPS, FX_FORM_CACHED, FX_FORM_TWO_CELLS, FX_FORM_LINEAR = 1, 2, 4, 8
+FX_FORM_XCD_ROWS, FX_FORM_BUFFER, FX_FORM_OFFSETS32 = 16, 32, 64
 FX_FIELD_FI, FX_FIELD_RHO_U_FLAGS, FX_FIELD_FLAGS, FX_FIELD_F = 0, 1, 2, 3
 
 STORAGE = {"FP32": FX_FP32, "FP16S": FX_FP16S, "FP16C": FX_FP16C}
@@ -42,6 +44,7 @@ EXPORTS = [
     "fx_adjoint_destroy", "fx_lbm_forward", "fx_lbm_backward", "fx_lbm_stream_collide_record", "fx_lbm_adjoint_step",
     "fx_lbm_objective_plane", "fx_transfer_bytes", "fx_lbm_transfer_extract", "fx_lbm_transfer_insert",
     "fx_lbm_update_moving_boundaries", "fx_buf_read_box", "fx_buf_write_box", "fx_lbm_mass_sum_noalloc",
+    "fx_ctx_launches",
 ]
 
 
@@ -54,6 +57,11 @@ class Config(ctypes.Structure):
 class AdjointConfig(ctypes.Structure):
     _fields_ = [("steps", ctypes.c_uint64), ("checkpoint_interval", ctypes.c_uint64), ("window_begin", ctypes.c_uint64),
                 ("plane_x", ctypes.c_uint32)]
+
+
+class Launches(ctypes.Structure):
+    _fields_ = [("one_step", ctypes.c_uint64), ("two_steps", ctypes.c_uint64), ("step_form", ctypes.c_uint32),
+                ("fields_form", ctypes.c_uint32), ("record_form", ctypes.c_uint32), ("adjoint_form", ctypes.c_uint32)]
 
 
 class DeviceInfo(ctypes.Structure):
@@ -92,6 +100,7 @@ def load():
     L.fx_ctx_create.argtypes = [i32, ctypes.POINTER(Config), ctypes.POINTER(vp)]
     L.fx_ctx_destroy.argtypes = [vp]
     L.fx_ctx_config.argtypes = [vp, ctypes.POINTER(Config)]
+    L.fx_ctx_launches.argtypes = [vp, ctypes.POINTER(Launches)]
     L.fx_sync.argtypes = [vp]
     L.fx_buf_alloc.argtypes = [vp, u64, ctypes.POINTER(vp)]
     L.fx_buf_free.argtypes = [vp, vp]
@@ -197,6 +206,12 @@ class Context:
             self.close()
         except Exception:
             pass
+
+    def launches(self):
+        """What the context launched for time steps so far (fx_ctx_launches)."""
+        out = Launches()
+        check(self.lib.fx_ctx_launches(self.h, ctypes.byref(out)))
+        return out
 
     def alloc(self, nbytes):
         p = ctypes.c_void_p()

@@ -6,6 +6,7 @@
 #include <cstring>
 #include <cmath>
 #include <string>
+#include <atomic>
 #include <mutex>
 #include <algorithm>
 #include <set>
@@ -54,6 +55,9 @@ struct fx_ctx {
 	fx::TwoStepShape shape_two{}; // two_steps launches of fx_lbm_run and fx_lbm_forward
 	void* second = nullptr;    // DDF array that two_steps launches alternate with (SecondArray)
 	bool second_busy = false;  // a call is queueing launches on it
+	// what fx_ctx_launches reports; calls from several threads may write them
+	std::atomic<uint64_t> one_step{0}, two_steps{0};
+	std::atomic<uint32_t> step_form{0}, fields_form{0}, record_form{0}, adjoint_form{0};
 };
 
 struct fx_adjoint {
@@ -195,6 +199,30 @@ struct SecondArray {
 	SecondArray& operator=(const SecondArray&) = delete;
 };
 
+uint32_t form_of(const fx::LaunchShape& s) {
+	return (s.cached ? FX_FORM_CACHED : 0u) | (s.pairs ? FX_FORM_TWO_CELLS : 0u) | (s.lin ? FX_FORM_LINEAR : 0u) | (s.xchunks ? FX_FORM_XCD_ROWS : 0u) |
+	       (s.buf ? FX_FORM_BUFFER : 0u) | (s.off32 ? FX_FORM_OFFSETS32 : 0u);
+}
+void launch_one_step(fx_ctx* ctx, const fx::LbmArgs& a) {
+	ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+	ctx->one_step++;
+	ctx->step_form = form_of(ctx->shape_sc);
+}
+void launch_two_steps(fx_ctx* ctx, const fx::LbmArgs& a, void* dst) {
+	ctx->k->two_steps(a, dst, ctx->shape_two, ctx->stream);
+	ctx->two_steps++;
+	ctx->step_form = FX_FORM_TWO_STEPS | (ctx->shape_two.cached ? FX_FORM_CACHED : 0u);
+}
+
+void launch_record(fx_ctx* ctx, const fx::LbmArgs& a, float* moments, void* dst) {
+	ctx->k->stream_collide_record(a, ctx->shape_rec, ctx->stream, moments, dst);
+	ctx->record_form = form_of(ctx->shape_rec);
+}
+void launch_adjoint_step(fx_ctx* ctx, const fx::AdjointArgs& g) {
+	ctx->k->adjoint_step(g, ctx->shape_adj, ctx->stream);
+	ctx->adjoint_form = form_of(ctx->shape_adj);
+}
+
 // Queues steps t .. t+steps-1 on a.fi.  Pairs of two_steps launches, fi -> second -> fi, take
 // four steps each and leave the DDFs where they were; the rest are single steps.
 void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps) {
@@ -205,16 +233,16 @@ void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps) {
 			a.odd = (uint32_t)(t & 1ull);
 			for(; steps >= 4u; steps -= 4u, t += 4u) {
 				a.fi = fi;
-				ctx->k->two_steps(a, second.array, ctx->shape_two, ctx->stream);
+				launch_two_steps(ctx, a, second.array);
 				a.fi = second.array;
-				ctx->k->two_steps(a, fi, ctx->shape_two, ctx->stream);
+				launch_two_steps(ctx, a, fi);
 			}
 			a.fi = fi;
 		}
 	}
 	for(; steps > 0u; steps--, t++) {
 		a.odd = (uint32_t)(t & 1ull);
-		ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+		launch_one_step(ctx, a);
 	}
 }
 
@@ -703,6 +731,13 @@ int fx_ctx_config(const fx_ctx* ctx, fx_lbm_config* out) {
 	return FX_OK;
 }
 
+int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out) {
+	if(!ctx || !out) return fail(FX_ERR_ARG, "null argument");
+	out->one_step = ctx->one_step; out->two_steps = ctx->two_steps;
+	out->step_form = ctx->step_form; out->fields_form = ctx->fields_form; out->record_form = ctx->record_form; out->adjoint_form = ctx->adjoint_form;
+	return FX_OK;
+}
+
 int fx_sync(fx_ctx* ctx) {
 	if(!ctx) return fail(FX_ERR_ARG, "null context");
 	FX_HIP(hipStreamSynchronize(ctx->stream));
@@ -793,8 +828,7 @@ int fx_lbm_stream_collide(fx_ctx* ctx, void* fi, float* rho, float* u, const uin
 	const int rc = check_step_args(ctx, fi, rho, u, flags, F, alpha);
 	if(rc != FX_OK) return rc;
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	const fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha);
-	ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+	launch_one_step(ctx, make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha));
 	return check_launch("stream_collide");
 }
 
@@ -823,6 +857,7 @@ int fx_lbm_update_fields(fx_ctx* ctx, const void* fi, float* rho, float* u, cons
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
 	const fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha);
 	ctx->k->update_fields(a, ctx->shape_uf, ctx->stream);
+	ctx->fields_form = form_of(ctx->shape_uf);
 	return check_launch("update_fields");
 }
 
@@ -974,7 +1009,7 @@ int fx_lbm_stream_collide_record(fx_ctx* ctx, void* fi, float* rho, float* u, co
 	if(ctx->cfg.extensions & (FX_MOVING_BOUNDARIES | FX_SUBGRID))
 		return fail(FX_ERR_CONFIG, "the adjoint does not differentiate MOVING_BOUNDARIES or SUBGRID");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	ctx->k->stream_collide_record(make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), ctx->shape_rec, ctx->stream, moments, fi);
+	launch_record(ctx, make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), moments, fi);
 	return check_launch("stream_collide_record");
 }
 
@@ -999,7 +1034,7 @@ int fx_lbm_adjoint_step(fx_ctx* ctx, float* lambda, const float* rho, const floa
 	if((ctx->cfg.extensions & FX_POROSITY) && !grad_alpha) return fail(FX_ERR_ARG, "POROSITY needs grad_alpha");
 	if((ctx->cfg.extensions & FX_EQUILIBRIUM_BOUNDARIES) && (!rho || !u)) return fail(FX_ERR_ARG, "TYPE_E presets rho/u required");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	ctx->k->adjoint_step(adjoint_args(ctx, lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, moments, plane_x, obj_weight, grad_alpha), ctx->shape_adj, ctx->stream);
+	launch_adjoint_step(ctx, adjoint_args(ctx, lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, moments, plane_x, obj_weight, grad_alpha));
 	return check_launch("adjoint_step");
 }
 
@@ -1068,7 +1103,7 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 			void* const end = n % 2u == 0u && (t + n) % adj->k == 0u ? (char*)saved + adj->fi_bytes : fi;
 			for(uint64_t left = pairs; left-- > 0u;) {
 				now = left == 0u ? end : (left & 1u) ? second.array : fi;
-				ctx->k->two_steps(b, now, ctx->shape_two, ctx->stream);
+				launch_two_steps(ctx, b, now);
 				b.fi = now;
 			}
 		} else if(now != fi) {
@@ -1114,13 +1149,13 @@ int fx_lbm_backward(fx_ctx* ctx, fx_adjoint* adj, const float* rho, const float*
 		for(uint64_t t = ts; t < te; t++) { // the first step from the checkpoint, which stays
 			a.fi = t == ts ? (void*)(adj->ckpt + s * adj->fi_bytes) : adj->work_fi;
 			a.odd = (uint32_t)(t & 1u);
-			ctx->k->stream_collide_record(a, ctx->shape_rec, ctx->stream, adj->moments + (t - ts) * 4u * N, adj->work_fi);
+			launch_record(ctx, a, adj->moments + (t - ts) * 4u * N, adj->work_fi);
 		}
 		for(uint64_t t = te; t-- > ts;) {
 			fx::AdjointArgs g = adjoint_args(ctx, adj->lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, adj->moments + (t - ts) * 4u * N,
 			                                 c.plane_x, t >= c.window_begin ? wobj : 0.0f, grad_alpha);
 			g.a.ext &= ~FX_UPDATE_FIELDS;
-			ctx->k->adjoint_step(g, ctx->shape_adj, ctx->stream);
+			launch_adjoint_step(ctx, g);
 		}
 		rc = check_launch("backward");
 		if(rc != FX_OK) return rc;

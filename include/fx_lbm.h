@@ -127,6 +127,21 @@ uint64_t fx_bandwidth_bytes_per_cell(const fx_lbm_config* cfg);
 int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out);
 int fx_ctx_destroy(fx_ctx* ctx);
 int fx_ctx_config(const fx_ctx* ctx, fx_lbm_config* out);
+/* What the context launched for time steps since it was created: launches that took one step
+ * (each reads and writes every DDF once) and launches that took two; and the form of the last
+ * launch of stream_collide, update_fields, the adjoint's record pass and the adjoint step. */
+#define FX_FORM_TWO_STEPS 1u /* two time steps per launch */
+#define FX_FORM_CACHED 2u    /* accesses that keep the DDFs in the caches; one cell per lane: on the cell-linear grid */
+#define FX_FORM_TWO_CELLS 4u /* two cells per lane */
+#define FX_FORM_LINEAR 8u    /* cell-linear grid; otherwise rows */
+#define FX_FORM_XCD_ROWS 16u /* rows of several blocks, each row on one XCD */
+#define FX_FORM_BUFFER 32u   /* buffer instructions allowed (DDFs below 4 GiB); kernels without them ignore it */
+#define FX_FORM_OFFSETS32 64u /* 32-bit slot offsets */
+typedef struct fx_launches {
+    uint64_t one_step, two_steps;
+    uint32_t step_form, fields_form, record_form, adjoint_form;
+} fx_launches;
+int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out);
 /* Wait for all work on the context stream; replaces Device::finish_queue (src/opencl.hpp:335). */
 int fx_sync(fx_ctx* ctx);
 
