@@ -44,7 +44,7 @@ EXPORTS = [
     "fx_adjoint_destroy", "fx_lbm_forward", "fx_lbm_backward", "fx_lbm_stream_collide_record", "fx_lbm_adjoint_step",
     "fx_lbm_objective_plane", "fx_transfer_bytes", "fx_lbm_transfer_extract", "fx_lbm_transfer_insert",
     "fx_lbm_update_moving_boundaries", "fx_buf_read_box", "fx_buf_write_box", "fx_lbm_mass_sum_noalloc",
-    "fx_ctx_launches",
+    "fx_ctx_launches", "fx_ctx_second_array", "fx_ctx_second_array_bytes",
 ]
 
 
@@ -101,6 +101,8 @@ def load():
     L.fx_ctx_destroy.argtypes = [vp]
     L.fx_ctx_config.argtypes = [vp, ctypes.POINTER(Config)]
     L.fx_ctx_launches.argtypes = [vp, ctypes.POINTER(Launches)]
+    L.fx_ctx_second_array.argtypes = [vp, i32]
+    L.fx_ctx_second_array_bytes.argtypes = [vp, ctypes.POINTER(u64), ctypes.POINTER(u64)]
     L.fx_sync.argtypes = [vp]
     L.fx_buf_alloc.argtypes = [vp, u64, ctypes.POINTER(vp)]
     L.fx_buf_free.argtypes = [vp, vp]
@@ -212,6 +214,17 @@ class Context:
         out = Launches()
         check(self.lib.fx_ctx_launches(self.h, ctypes.byref(out)))
         return out
+
+    def set_second_array(self, allowed):
+        """Whether runs may take a second DDF array for launches of two steps; False also
+        gives back the one that the context holds (fx_ctx_second_array)."""
+        check(self.lib.fx_ctx_second_array(self.h, 1 if allowed else 0))
+
+    def second_array_bytes(self):
+        """(bytes of the second DDF array held now, bytes that a run may take)."""
+        held, most = ctypes.c_uint64(), ctypes.c_uint64()
+        check(self.lib.fx_ctx_second_array_bytes(self.h, ctypes.byref(held), ctypes.byref(most)))
+        return held.value, most.value
 
     def alloc(self, nbytes):
         p = ctypes.c_void_p()

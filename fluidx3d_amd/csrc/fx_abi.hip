@@ -55,6 +55,7 @@ struct fx_ctx {
 	fx::TwoStepShape shape_two{}; // two_steps launches of fx_lbm_run and fx_lbm_forward
 	void* second = nullptr;    // DDF array that two_steps launches alternate with (SecondArray)
 	bool second_busy = false;  // a call is queueing launches on it
+	bool second_allowed = true; // fx_ctx_second_array
 	// what fx_ctx_launches reports; calls from several threads may write them
 	std::atomic<uint64_t> one_step{0}, two_steps{0};
 	std::atomic<uint32_t> step_form{0}, fields_form{0}, record_form{0}, adjoint_form{0};
@@ -113,12 +114,12 @@ uint64_t ddf_bytes(const fx_ctx* ctx) {
 // ---- second DDF arrays ----
 // two_steps launches read one DDF array and write another.  The second one belongs to the
 // context that runs them and is allocated by its first run that can use it, if at least half
-// of the device memory stays free; it is kept for the next run, and given back when any
-// context of the device cannot allocate what its caller asked for (allocate_device), or with
-// the context.  Launches on one context's stream run in order, so the next call may use the
+// of the device memory stays free and the caller did not decline it (fx_ctx_second_array); it is
+// kept for the next run, and given back when the caller asks for that, when any context of the
+// device cannot allocate what its caller asked for (allocate_device), or with the context.  Launches on one context's stream run in order, so the next call may use the
 // array while the last one's launches still run; a call from another thread that comes while
 // one is queueing takes single steps.  g_second_mutex guards the list and every context's
-// `second` and `second_busy`.
+// `second`, `second_busy` and `second_allowed`.
 std::mutex g_second_mutex;
 std::set<fx_ctx*> g_second_owners;
 
@@ -179,7 +180,7 @@ struct SecondArray {
 	explicit SecondArray(fx_ctx* c, bool wanted = true) : ctx(c) {
 		if(!wanted) return;
 		std::lock_guard<std::mutex> lock(g_second_mutex);
-		if(ctx->second_busy) return; // another thread is queueing launches on it
+		if(!ctx->second_allowed || ctx->second_busy) return; // busy: another thread is queueing launches on it
 		if(!ctx->second) {
 			const RelaxedCapture relaxed;
 			size_t f = 0, total = 0;
@@ -194,6 +195,7 @@ struct SecondArray {
 		if(!array) return;
 		std::lock_guard<std::mutex> lock(g_second_mutex);
 		ctx->second_busy = false;
+		if(!ctx->second_allowed) release_second_locked(ctx); // declined in the meantime
 	}
 	SecondArray(const SecondArray&) = delete;
 	SecondArray& operator=(const SecondArray&) = delete;
@@ -735,6 +737,23 @@ int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out) {
 	if(!ctx || !out) return fail(FX_ERR_ARG, "null argument");
 	out->one_step = ctx->one_step; out->two_steps = ctx->two_steps;
 	out->step_form = ctx->step_form; out->fields_form = ctx->fields_form; out->record_form = ctx->record_form; out->adjoint_form = ctx->adjoint_form;
+	return FX_OK;
+}
+
+int fx_ctx_second_array(fx_ctx* ctx, int allowed) {
+	if(!ctx) return fail(FX_ERR_ARG, "null context");
+	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
+	std::lock_guard<std::mutex> lock(g_second_mutex);
+	ctx->second_allowed = allowed != 0;
+	if(!allowed && !ctx->second_busy) release_second_locked(ctx); // busy: that call gives it back (SecondArray)
+	return FX_OK;
+}
+
+int fx_ctx_second_array_bytes(const fx_ctx* ctx, uint64_t* held, uint64_t* most) {
+	if(!ctx) return fail(FX_ERR_ARG, "null context");
+	std::lock_guard<std::mutex> lock(g_second_mutex);
+	if(held) *held = ctx->second ? ddf_bytes(ctx) : 0u;
+	if(most) *most = ctx->shape_two.grid ? ddf_bytes(ctx) : 0u;
 	return FX_OK;
 }
 

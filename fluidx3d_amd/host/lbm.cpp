@@ -393,6 +393,9 @@ void LBM::update_fields() {
 }
 
 void LBM::reset() { initialized = false; }
+void LBM::set_second_array(const bool allowed) {
+	for(uint d = 0u; d < get_D(); d++) fx_check(fx_ctx_second_array(domain[d].ctx, allowed ? 1 : 0), "second_array");
+}
 
 // DDF codes as the kernels store them (src/lbm.cpp:410-414, src/kernel.cpp:848-859), for
 // the host-side sum over the interior cells of split lattices

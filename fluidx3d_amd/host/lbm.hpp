@@ -156,6 +156,7 @@ public:
 	void update_moving_boundaries(); // mark/unmark cells next to TYPE_S cells with velocity!=0 with TYPE_MS
 #endif
 	void reset();         // next run() re-initializes from the host fields
+	void set_second_array(const bool allowed); // false: run() holds no second DDF array (fx_ctx_second_array)
 #ifdef FORCE_FIELD
 	void update_force_field();
 	float3 object_center_of_mass(const uchar flag_marker = TYPE_S);

@@ -191,6 +191,11 @@ class LBM:
             self.t_last_update_fields = self.t
         self.ctx.sync()
 
+    def set_second_array(self, allowed):
+        """Runs of FP32 lattices may hold a second DDF array (q*N*4 bytes) for launches of two
+        steps; False gives it back and keeps further runs from taking one, same results."""
+        self.ctx.set_second_array(allowed)
+
     def _update_fields_if_stale(self):
         if self.t_last_update_fields != self.t:
             check(self.ctx.lib.fx_lbm_update_fields(*self._step_args(), self.t, self.fx, self.fy, self.fz,

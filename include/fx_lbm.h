@@ -142,6 +142,14 @@ typedef struct fx_launches {
     uint32_t step_form, fields_form, record_form, adjoint_form;
 } fx_launches;
 int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out);
+/* The second DDF array of fx_lbm_run's launches of two steps (see there): device memory beside
+ * the caller's buffers and the byte counts above.  allowed == 0 gives it back, after waiting for
+ * the context's work, and keeps further runs from taking one (they take single steps, the same
+ * bits); allowed != 0, the default, lets the next run take one again.  held: bytes the context
+ * holds now; most: bytes it may come to hold (0 where the lattice takes no such launches);
+ * either may be NULL. */
+int fx_ctx_second_array(fx_ctx* ctx, int allowed);
+int fx_ctx_second_array_bytes(const fx_ctx* ctx, uint64_t* held, uint64_t* most);
 /* Wait for all work on the context stream; replaces Device::finish_queue (src/opencl.hpp:335). */
 int fx_sync(fx_ctx* ctx);
 
@@ -197,8 +205,10 @@ int fx_lbm_stream_collide(fx_ctx* ctx, void* fi, float* rho, float* u, const uin
  * not NULL bracketed by HIP events, and the call waits and returns the elapsed milliseconds.
  * FP32 lattices on which it is faster take two steps per launch, with a second DDF array that the
  * context allocates once if half of the device memory stays free, keeps, and gives back when an
- * allocation through this interface would fail without it; otherwise, and with an array that
- * cannot be had, each step is a stream_collide launch.  The results are the same bits.
+ * allocation through this interface would fail without it or fx_ctx_second_array asks for it;
+ * otherwise, and with an array that cannot be had, each step is a stream_collide launch.
+ * Allocators outside this interface cannot reclaim the array: a program that shares the device
+ * with one (torch, another process) sizes it in, or declines it.  The results are the same bits.
  * Replaces the loop of LBM::run (src/lbm.cpp:955-975) without the per-step host
  * synchronisation of src/lbm.cpp:951. */
 int fx_lbm_run(fx_ctx* ctx, void* fi, float* rho, float* u, const uint8_t* flags, uint64_t t0, uint64_t steps,

@@ -1,0 +1,55 @@
+"""The second DDF array that FP32 runs of several steps hold for launches of two steps: taken by
+the first run that can use it, counted, declined and given back by the caller
+(fx_ctx_second_array), with the same bits either way."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tests.test_two_steps import scene_lbm, single_steps
+
+pytestmark = pytest.mark.gpu
+SIZE = (128, 96, 96)  # 86 MiB of DDFs, a lattice that takes two steps per launch
+
+
+def test_declined_and_given_back():
+    import fluidx3d_amd as fx
+    a, b = (scene_lbm(fx, SIZE, 19, "SRT", ()) for _ in range(2))
+    array = 19 * a.N * 4
+    try:
+        def run(steps):
+            before = a.ctx.launches()
+            a.run(steps)
+            single_steps(b, steps)
+            assert np.array_equal(a.read_ddfs().view(np.uint32), b.read_ddfs().view(np.uint32))
+            after = a.ctx.launches()
+            return after.one_step - before.one_step, after.two_steps - before.two_steps
+
+        assert a.ctx.second_array_bytes() == (0, array)
+        assert run(3) == (3, 0) and a.ctx.second_array_bytes() == (0, array)
+        assert run(9) == (1, 4) and a.ctx.second_array_bytes() == (array, array)
+        held = fx.device_info(0)["memory_free"]
+        a.set_second_array(False)
+        assert a.ctx.second_array_bytes() == (0, array)
+        assert fx.device_info(0)["memory_free"] - held >= array
+        assert run(8) == (8, 0) and a.ctx.second_array_bytes() == (0, array)
+        a.set_second_array(True)
+        assert a.ctx.second_array_bytes() == (0, array)
+        assert run(8) == (0, 4) and a.ctx.second_array_bytes() == (array, array)
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("size,storage", [((64, 64, 64), "FP32"), (SIZE, "FP16S")])
+def test_lattices_without_one(size, storage):
+    import fluidx3d_amd as fx
+    lbm = fx.LBM(*size, 0.05, storage=storage)
+    try:
+        lbm.run(8)
+        assert lbm.ctx.second_array_bytes() == (0, 0) and lbm.ctx.launches().two_steps == 0
+        lbm.set_second_array(False)
+        assert lbm.ctx.lib.fx_ctx_second_array_bytes(lbm.ctx.h, None, None) == 0
+        assert lbm.ctx.lib.fx_ctx_second_array_bytes(None, None, ctypes.byref(ctypes.c_uint64())) == -1
+    finally:
+        lbm.close()
