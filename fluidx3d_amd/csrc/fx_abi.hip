@@ -53,7 +53,7 @@ struct fx_ctx {
 	double* scratch = nullptr; // this device's copy of the static scratch array (fx_lbm_mass_sum_noalloc)
 	std::set<void*> buffers;   // allocations owned by this context
 	fx::TwoStepShape shape_two{}; // two_steps launches of fx_lbm_run and fx_lbm_forward
-	void* second = nullptr;    // DDF array that two_steps launches alternate with (SecondArray)
+	void* second = nullptr;    // DDF array that fx_lbm_run's two_steps launches alternate with (SecondArray)
 	bool second_busy = false;  // a call is queueing launches on it
 	bool second_allowed = true; // fx_ctx_second_array
 	// what fx_ctx_launches reports; calls from several threads may write them
@@ -66,7 +66,7 @@ struct fx_adjoint {
 	fx_adjoint_config cfg{};
 	uint64_t k = 0, checkpoints = 0, fi_bytes = 0, obj_blocks = 0;
 	char* ckpt = nullptr;       // checkpoints * fi_bytes
-	void* work_fi = nullptr;    // recomputation state
+	void* work_fi = nullptr;    // recomputation state; in the forward pass, the other array of the two_steps launches
 	float* moments = nullptr;   // k * 4 * N
 	float* lambda = nullptr;    // q * N
 	double* acc = nullptr;      // 1
@@ -177,8 +177,7 @@ int ensure_partial(fx_ctx* ctx, uint64_t doubles) {
 struct SecondArray {
 	fx_ctx* ctx;
 	void* array = nullptr;
-	explicit SecondArray(fx_ctx* c, bool wanted = true) : ctx(c) {
-		if(!wanted) return;
+	explicit SecondArray(fx_ctx* c) : ctx(c) {
 		std::lock_guard<std::mutex> lock(g_second_mutex);
 		if(!ctx->second_allowed || ctx->second_busy) return; // busy: another thread is queueing launches on it
 		if(!ctx->second) {
@@ -1096,9 +1095,8 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 		summed = 0;
 	};
 	// Before the window every span of steps runs from one checkpoint to the next or to the
-	// window: pairs of steps from the checkpoint, fi and the second array in turn, to the next
-	// checkpoint, so that no copy of the DDFs is made.
-	const SecondArray second(ctx, ctx->shape_two.grid && adj->k >= 2u && c.window_begin >= 2u);
+	// window: pairs of steps from the checkpoint, fi and work_fi (the backward sweep's) in turn, to
+	// the next checkpoint, so that no copy of the DDFs is made.
 	void* now = fi; // the state of step t
 	for(uint64_t t = 0, n = 0; t < c.steps; t += n) {
 		void* const saved = adj->ckpt + (t / adj->k) * adj->fi_bytes;
@@ -1109,19 +1107,19 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 			a.odd = (uint32_t)(t & 1u);
 			ctx->k->objective_partial(a, c.plane_x, ctx->stream, partial + summed * adj->obj_blocks);
 			if(++summed == batch) sum_objective();
-			queue_steps(ctx, a, t, 1u);
+			launch_one_step(ctx, a);
 			n = 1u; // the objective looks at every step
 			continue;
 		}
 		n = std::min(adj->k - t % adj->k, c.window_begin - t); // up to the next checkpoint or the window (window_begin < steps)
-		const uint64_t pairs = second.array ? n / 2u : 0u;
+		const uint64_t pairs = ctx->shape_two.grid ? n / 2u : 0u;
 		fx::LbmArgs b = a;
 		b.odd = (uint32_t)(t & 1u);
 		if(pairs > 0u) {
 			b.fi = saved;
 			void* const end = n % 2u == 0u && (t + n) % adj->k == 0u ? (char*)saved + adj->fi_bytes : fi;
 			for(uint64_t left = pairs; left-- > 0u;) {
-				now = left == 0u ? end : (left & 1u) ? second.array : fi;
+				now = left == 0u ? end : (left & 1u) ? adj->work_fi : fi;
 				launch_two_steps(ctx, b, now);
 				b.fi = now;
 			}
@@ -1129,7 +1127,10 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 			FX_HIP(hipMemcpyAsync(fi, now, adj->fi_bytes, hipMemcpyDeviceToDevice, ctx->stream));
 			now = fi;
 		}
-		queue_steps(ctx, a, t + 2u * pairs, n - 2u * pairs);
+		for(uint64_t s = t + 2u * pairs; s < t + n; s++) {
+			a.odd = (uint32_t)(s & 1u);
+			launch_one_step(ctx, a);
+		}
 	}
 	if(summed > 0u) sum_objective();
 	rc = check_launch("forward");

@@ -278,7 +278,7 @@ int fx_adjoint_memory(const fx_ctx* ctx, const fx_adjoint_config* cfg, uint64_t*
 int fx_adjoint_create(fx_ctx* ctx, const fx_adjoint_config* cfg, fx_adjoint** out);
 int fx_adjoint_destroy(fx_adjoint* adj);
 /* forward pass with checkpoints; *objective = J; *ms = GPU time (either may be NULL).  Steps
- * before the window go two per launch where fx_lbm_run's do */
+ * before the window go two per launch where fx_lbm_run's do, within adj's workspace */
 int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u, const uint8_t* flags,
                    float fx, float fy, float fz, const float* F, const float* alpha, double* objective, float* ms);
 /* checkpointed adjoint sweep after fx_lbm_forward; rho/u hold the TYPE_E presets */

@@ -53,3 +53,28 @@ def test_lattices_without_one(size, storage):
         assert lbm.ctx.lib.fx_ctx_second_array_bytes(None, None, ctypes.byref(ctypes.c_uint64())) == -1
     finally:
         lbm.close()
+
+
+def test_adjoint_forward_takes_none():
+    """Adjoint.forward alternates with the workspace's own array: two steps per launch, no
+    device memory beyond the workspace, also where the second array is declined."""
+    import fluidx3d_amd as fx
+    from fluidx3d_amd.adjoint import Adjoint
+    from tests import scenes
+    rho, u, flags, alpha = scenes.porous_channel(128, 64, 58)
+    results = []
+    for allowed in (True, False):
+        lbm = fx.LBM(128, 64, 58, 1.0 / 6.0, 1e-5, 0.0, 0.0, extensions=("VOLUME_FORCE", "POROSITY", "PRECISE_DENSITY"))
+        try:
+            lbm.set_second_array(allowed)
+            lbm.rho.host[:], lbm.u.host[:], lbm.flags.host[:], lbm.porosity.host[:] = rho, u, flags, alpha
+            adj = Adjoint(lbm, steps=31, window_begin=24, plane_x=127, checkpoint_interval=8)
+            results.append((adj.forward(), lbm.read_ddfs(), adj.backward()))
+            n = lbm.ctx.launches()
+            assert (n.two_steps, n.one_step) == (12, 7)
+            assert lbm.ctx.second_array_bytes() == (0, 19 * lbm.N * 4)
+            adj.close()
+        finally:
+            lbm.close()
+    for a, b in zip(*results):
+        assert np.array_equal(a, b)
