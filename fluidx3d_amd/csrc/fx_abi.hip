@@ -113,8 +113,8 @@ uint64_t ddf_bytes(const fx_ctx* ctx) {
 
 // ---- second DDF arrays ----
 // two_steps launches read one DDF array and write another.  The second one belongs to the
-// context that runs them and is allocated by its first run that can use it, if at least half
-// of the device memory stays free and the caller did not decline it (fx_ctx_second_array); it is
+// context that runs them and is allocated by its first run that can use it, if there is room
+// (second_array_fits) and the caller did not decline it (fx_ctx_second_array); it is
 // kept for the next run, and given back when the caller asks for that, when any context of the
 // device cannot allocate what its caller asked for (allocate_device), or with the context.  Launches on one context's stream run in order, so the next call may use the
 // array while the last one's launches still run; a call from another thread that comes while
@@ -184,7 +184,7 @@ struct SecondArray {
 		if(!ctx->second) {
 			const RelaxedCapture relaxed;
 			size_t f = 0, total = 0;
-			if(hipMemGetInfo(&f, &total) != hipSuccess || ddf_bytes(ctx) + total / 2u > f) { (void)hipGetLastError(); return; }
+			if(hipMemGetInfo(&f, &total) != hipSuccess || !fx::second_array_fits(ddf_bytes(ctx), f, total)) { (void)hipGetLastError(); return; }
 			if(hipMalloc(&ctx->second, ddf_bytes(ctx)) != hipSuccess) { (void)hipGetLastError(); ctx->second = nullptr; return; }
 			g_second_owners.insert(ctx);
 		}

@@ -378,6 +378,12 @@ inline bool two_steps_pay(const TwoStepShape& s, uint32_t Nx, uint32_t Ny, uint3
 	return percent >= (weight > 2u ? 90u : s.wide ? 55u : 40u);
 }
 
+// Whether fx_lbm_run takes a second DDF array of `bytes`: half of the device stays free beside
+// it, or it is a small part of what is free (other programs may hold most of the device).
+inline bool second_array_fits(uint64_t bytes, uint64_t free_bytes, uint64_t total_bytes) {
+	return bytes <= free_bytes / 16u || (bytes <= free_bytes && free_bytes - bytes >= total_bytes / 2u);
+}
+
 // Kernel set of one (velocity set, storage, collision) variant; EXT = 0 instantiates the
 // extension-free kernels, EXT_ALL the ones that read the runtime extension mask.
 template<int Q, uint32_t ST, bool TRT, uint32_t EXT> struct KernelSet {

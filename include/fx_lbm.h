@@ -204,7 +204,8 @@ int fx_lbm_stream_collide(fx_ctx* ctx, void* fi, float* rho, float* u, const uin
 /* The time steps t = t0 .. t0+steps-1, queued back to back on the context stream; with ms
  * not NULL bracketed by HIP events, and the call waits and returns the elapsed milliseconds.
  * FP32 lattices on which it is faster take two steps per launch, with a second DDF array that the
- * context allocates once if half of the device memory stays free, keeps, and gives back when an
+ * context allocates once if half of the device memory stays free or the array is at most a
+ * sixteenth of what is free, keeps, and gives back when an
  * allocation through this interface would fail without it or fx_ctx_second_array asks for it;
  * otherwise, and with an array that cannot be had, each step is a stream_collide launch.
  * Allocators outside this interface cannot reclaim the array: a program that shares the device
