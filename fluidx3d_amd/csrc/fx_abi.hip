@@ -21,7 +21,10 @@ int fail(int code, const std::string& message) {
 	g_last_error = message;
 	return code;
 }
+// The runtime keeps the error of a failed call until it is asked for: without the question, the
+// next launch's check_launch would report it.
 int fail_hip(hipError_t e, const char* what) {
+	(void)hipGetLastError();
 	return fail(FX_ERR_HIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 #define FX_HIP(call) do { const hipError_t fx_e_ = (call); if(fx_e_ != hipSuccess) return fail_hip(fx_e_, #call); } while(0)
@@ -153,6 +156,7 @@ hipError_t allocate_device(int device, void** p, uint64_t bytes) {
 		(void)hipGetLastError();
 		e = hipMalloc(p, bytes);
 	}
+	if(e != hipSuccess) (void)hipGetLastError(); // see fail_hip
 	return e;
 }
 // Free memory of the current device, counting second arrays that would be given back.

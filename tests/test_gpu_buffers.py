@@ -107,3 +107,20 @@ def test_box_argument_errors():
             lbm.u.read_from_device_2d(0, 4, 0, 2, 0, 2)                # Nx = 0
     finally:
         lbm.close()
+
+
+def test_failed_allocation_is_reported_once():
+    """An allocation that cannot be had is an FX_ERR_MEMORY of that call only; the next step
+    neither fails nor reports it."""
+    import fluidx3d_amd as fx
+    from fluidx3d_amd import _abi
+    lbm = fx.LBM(Nx, Ny, Nz, 0.05)
+    try:
+        lbm.run(1)
+        with pytest.raises(_abi.FxError) as e:
+            lbm.ctx.alloc(1 << 42)
+        assert e.value.code == _abi.FX_ERR_MEMORY
+        lbm.run(1)
+        assert lbm.t == 2
+    finally:
+        lbm.close()
