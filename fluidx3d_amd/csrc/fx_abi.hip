@@ -59,6 +59,7 @@ struct fx_ctx {
 	void* second = nullptr;    // DDF array that fx_lbm_run's two_steps launches alternate with (SecondArray)
 	bool second_busy = false;  // a call is queueing launches on it
 	bool second_allowed = true; // fx_ctx_second_array
+	fx_ctx* next = nullptr;    // g_contexts
 	// what fx_ctx_launches reports; calls from several threads may write them
 	std::atomic<uint64_t> one_step{0}, two_steps{0};
 	std::atomic<uint32_t> step_form{0}, fields_form{0}, record_form{0}, adjoint_form{0};
@@ -121,10 +122,11 @@ uint64_t ddf_bytes(const fx_ctx* ctx) {
 // kept for the next run, and given back when the caller asks for that, when any context of the
 // device cannot allocate what its caller asked for (allocate_device), or with the context.  Launches on one context's stream run in order, so the next call may use the
 // array while the last one's launches still run; a call from another thread that comes while
-// one is queueing takes single steps.  g_second_mutex guards the list and every context's
-// `second`, `second_busy` and `second_allowed`.
-std::mutex g_second_mutex;
-std::set<fx_ctx*> g_second_owners;
+// one is queueing takes single steps.  g_contexts_mutex guards the list of contexts (linked
+// through the contexts, so that a run allocates no host memory and cannot throw) and every
+// context's `second`, `second_busy` and `second_allowed`.
+std::mutex g_contexts_mutex;
+fx_ctx* g_contexts = nullptr;
 
 // Allocations must not disturb a stream capture that another library has open in this thread.
 struct RelaxedCapture {
@@ -139,15 +141,13 @@ void release_second_locked(fx_ctx* ctx) {
 	(void)hipStreamSynchronize(ctx->stream);
 	(void)hipFree(ctx->second);
 	ctx->second = nullptr;
-	g_second_owners.erase(ctx);
 }
 // Gives back every second array of the device that no call is using; true if there was one.
 bool release_second_arrays(int device) {
-	std::lock_guard<std::mutex> lock(g_second_mutex);
+	std::lock_guard<std::mutex> lock(g_contexts_mutex);
 	bool any = false;
-	const std::set<fx_ctx*> owners = g_second_owners;
-	for(fx_ctx* c : owners)
-		if(c->device == device && !c->second_busy) { release_second_locked(c); any = true; }
+	for(fx_ctx* c = g_contexts; c; c = c->next)
+		if(c->device == device && c->second && !c->second_busy) { release_second_locked(c); any = true; }
 	return any;
 }
 hipError_t allocate_device(int device, void** p, uint64_t bytes) {
@@ -183,21 +183,20 @@ struct SecondArray {
 	void* array = nullptr;
 	SecondArray(fx_ctx* c, bool wanted) : ctx(c) {
 		if(!wanted) return;
-		std::lock_guard<std::mutex> lock(g_second_mutex);
+		std::lock_guard<std::mutex> lock(g_contexts_mutex);
 		if(!ctx->second_allowed || ctx->second_busy) return; // busy: another thread is queueing launches on it
 		if(!ctx->second) {
 			const RelaxedCapture relaxed;
 			size_t f = 0, total = 0;
 			if(hipMemGetInfo(&f, &total) != hipSuccess || !fx::second_array_fits(ddf_bytes(ctx), f, total)) { (void)hipGetLastError(); return; }
 			if(hipMalloc(&ctx->second, ddf_bytes(ctx)) != hipSuccess) { (void)hipGetLastError(); ctx->second = nullptr; return; }
-			g_second_owners.insert(ctx);
 		}
 		ctx->second_busy = true;
 		array = ctx->second;
 	}
 	~SecondArray() {
 		if(!array) return;
-		std::lock_guard<std::mutex> lock(g_second_mutex);
+		std::lock_guard<std::mutex> lock(g_contexts_mutex);
 		ctx->second_busy = false;
 		if(!ctx->second_allowed) release_second_locked(ctx); // declined in the meantime
 	}
@@ -707,6 +706,11 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 		fx_ctx_destroy(ctx);
 		return fail(FX_ERR_HIP, msg);
 	}
+	{
+		std::lock_guard<std::mutex> lock(g_contexts_mutex);
+		ctx->next = g_contexts;
+		g_contexts = ctx;
+	}
 	*out = ctx;
 	return FX_OK;
 }
@@ -716,8 +720,9 @@ int fx_ctx_destroy(fx_ctx* ctx) {
 	(void)hipSetDevice(ctx->device);
 	if(ctx->stream) (void)hipStreamSynchronize(ctx->stream);
 	{
-		std::lock_guard<std::mutex> lock(g_second_mutex);
+		std::lock_guard<std::mutex> lock(g_contexts_mutex);
 		release_second_locked(ctx);
+		for(fx_ctx** c = &g_contexts; *c; c = &(*c)->next) if(*c == ctx) { *c = ctx->next; break; }
 	}
 	for(void* p : ctx->buffers) (void)hipFree(p);
 	if(ctx->partial) (void)hipFree(ctx->partial);
@@ -745,7 +750,7 @@ int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out) {
 int fx_ctx_second_array(fx_ctx* ctx, int allowed) {
 	if(!ctx) return fail(FX_ERR_ARG, "null context");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	std::lock_guard<std::mutex> lock(g_second_mutex);
+	std::lock_guard<std::mutex> lock(g_contexts_mutex);
 	ctx->second_allowed = allowed != 0;
 	if(!allowed && !ctx->second_busy) release_second_locked(ctx); // busy: that call gives it back (SecondArray)
 	return FX_OK;
@@ -753,7 +758,7 @@ int fx_ctx_second_array(fx_ctx* ctx, int allowed) {
 
 int fx_ctx_second_array_bytes(const fx_ctx* ctx, uint64_t* held, uint64_t* most) {
 	if(!ctx) return fail(FX_ERR_ARG, "null context");
-	std::lock_guard<std::mutex> lock(g_second_mutex);
+	std::lock_guard<std::mutex> lock(g_contexts_mutex);
 	if(held) *held = ctx->second ? ddf_bytes(ctx) : 0u;
 	if(most) *most = ctx->shape_two.grid ? ddf_bytes(ctx) : 0u;
 	return FX_OK;

@@ -1,7 +1,9 @@
 """The second DDF array when device memory is short.  hipMalloc and hipMemGetInfo are replaced
 on the host, in a process of its own: a small library, loaded before the HIP library with its
 symbols global, fails a chosen number of allocations of one size and reports a chosen amount of
-free memory.  Every allocation that it lets through is the runtime's."""
+free memory.  Every allocation that it lets through is the runtime's.  It also counts the host
+allocations (operator new) of libfx_lbm.so: a run makes none, so it cannot throw through the C
+interface."""
 import json
 import os
 import subprocess
@@ -13,9 +15,12 @@ pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 INTERPOSER = r'''
-#define _GNU_SOURCE
 #include <dlfcn.h>
 #include <stddef.h>
+#include <stdlib.h>
+#include <string.h>
+#include <new>
+extern "C" {
 static void* hip(const char* name) {
 	static void* lib = 0;
 	if(!lib) lib = dlopen("libamdhip64.so", RTLD_NOW | RTLD_LOCAL);
@@ -31,6 +36,17 @@ int hipMalloc(void** p, size_t n) {
 int hipMemGetInfo(size_t* f, size_t* t) {
 	if(fake_total) { *f = fake_free; *t = fake_total; return 0; }
 	return ((int (*)(size_t*, size_t*))hip("hipMemGetInfo"))(f, t);
+}
+int counting = 0, news = 0;
+}
+void* operator new(size_t n) {
+	if(counting) {
+		Dl_info i;
+		if(dladdr(__builtin_return_address(0), &i) && i.dli_fname && strstr(i.dli_fname, "libfx_lbm")) news++;
+	}
+	void* p = malloc(n ? n : 1);
+	if(!p) throw std::bad_alloc();
+	return p;
 }
 '''
 
@@ -49,7 +65,9 @@ a, b = (scene_lbm(fx, SIZE, 19, "SRT", ()) for _ in range(2))
 array = 19 * a.N * 4
 def run(steps):
     n = a.ctx.launches().two_steps
+    var("counting").value = 1
     a.run(steps)
+    var("counting").value = 0
     single_steps(b, steps)
     same = bool(np.array_equal(a.read_ddfs().view(np.uint32), b.read_ddfs().view(np.uint32)))
     return [a.ctx.launches().two_steps - n, a.ctx.second_array_bytes()[0] // array, same]
@@ -81,7 +99,13 @@ except _abi.FxError as e:
     out["refused"] = e.code == _abi.FX_ERR_MEMORY
 var("fail_count").value = 0
 out["then"] = run(5)
-a.close(); b.close()
+out["host allocations of the runs"] = var("news").value
+a.set_second_array(True)
+var("counting").value = 1
+c = scene_lbm(fx, SIZE, 19, "SRT", ())
+var("counting").value = 0
+out["counted"] = var("news").value > 0  # a context is allocated
+a.close(); b.close(); c.close()
 print(json.dumps(out))
 '''
 
@@ -89,8 +113,8 @@ print(json.dumps(out))
 @pytest.fixture(scope="module")
 def outcome(tmp_path_factory):
     d = tmp_path_factory.mktemp("interposer")
-    (d / "i.c").write_text(INTERPOSER)
-    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", str(d / "i.c"), "-o", str(d / "i.so"), "-ldl"], check=True)
+    (d / "i.cpp").write_text(INTERPOSER)
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", str(d / "i.cpp"), "-o", str(d / "i.so"), "-ldl"], check=True)
     r = subprocess.run([sys.executable, "-c", PROGRAM, str(d / "i.so")], cwd=ROOT, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0, r.stderr[-3000:]
     return json.loads(r.stdout.strip().splitlines()[-1])
@@ -99,6 +123,7 @@ def outcome(tmp_path_factory):
 # [launches of two steps, second arrays held, DDFs equal those of single steps, ...]
 @pytest.mark.parametrize("what,expected", [
     ("scarce", [0, 0, True]), ("small", [4, 1, True]), ("malloc fails", [0, 0, True, 1]), ("next run", [4, 1, True]),
-    ("given back", [0, 1, True]), ("after", [4, 1, True]), ("refused", True), ("then", [0, 0, True])])
+    ("given back", [0, 1, True]), ("after", [4, 1, True]), ("refused", True), ("then", [0, 0, True]),
+    ("host allocations of the runs", 0), ("counted", True)])
 def test_short_memory(outcome, what, expected):
     assert outcome[what] == expected, outcome
