@@ -45,8 +45,9 @@ struct fx_ctx {
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
 	const fx::LbmKernels* k = nullptr;
 	fx::Divisor by_Nx, by_Ny;
-	fx::LaunchShape shape{};    // one lane per cell: every kernel but stream_collide
+	fx::LaunchShape shape{};    // one lane per cell: every other lattice kernel
 	fx::LaunchShape shape_sc{}; // stream_collide (residency cap, XCD-mapped grid)
+	fx::LaunchShape shape_sc_crowded{}; // a single step whose DDFs other lattices drove from the cache (step_shape)
 	fx::LaunchShape shape_uf{};  // update_fields
 	fx::LaunchShape shape_rec{}; // the adjoint's record pass
 	fx::LaunchShape shape_adj{}; // adjoint step (XCD-mapped grid)
@@ -60,6 +61,8 @@ struct fx_ctx {
 	bool second_busy = false;  // a call is queueing launches on it
 	bool second_allowed = true; // fx_ctx_second_array
 	fx_ctx* next = nullptr;    // g_contexts
+	uint64_t touched = 0;      // g_touches when a call last went over the DDFs
+	bool reread = false;       // update_fields followed the last step
 	// what fx_ctx_launches reports; calls from several threads may write them
 	std::atomic<uint64_t> one_step{0}, two_steps{0};
 	std::atomic<uint32_t> step_form{0}, fields_form{0}, record_form{0}, adjoint_form{0};
@@ -124,7 +127,7 @@ uint64_t ddf_bytes(const fx_ctx* ctx) {
 // array while the last one's launches still run; a call from another thread that comes while
 // one is queueing takes single steps.  g_contexts_mutex guards the list of contexts (linked
 // through the contexts, so that a run allocates no host memory and cannot throw) and every
-// context's `second`, `second_busy` and `second_allowed`.
+// context's `second`, `second_busy`, `second_allowed`, `touched` and `reread`.
 std::mutex g_contexts_mutex;
 fx_ctx* g_contexts = nullptr;
 
@@ -204,14 +207,39 @@ struct SecondArray {
 	SecondArray& operator=(const SecondArray&) = delete;
 };
 
+// ---- lattices that share the last-level cache ----
+uint64_t g_touches = 0; // guarded by g_contexts_mutex
+
+// A call other than a step goes over the context's DDFs.
+void touch(fx_ctx* ctx, bool reread) {
+	std::lock_guard<std::mutex> lock(g_contexts_mutex);
+	ctx->touched = ++g_touches;
+	ctx->reread = reread;
+}
+// stream_collide's launch for `steps` steps.  A small lattice's DDFs are in the cache from one
+// step to the next, but before the first only if the lattices that the device's other contexts went
+// over since this one's last call left them there (crowds_cache).  A program that looks at the
+// fields after its single steps finds the DDFs of a cached one there.
+const fx::LaunchShape& step_shape(fx_ctx* ctx, uint64_t steps) {
+	std::lock_guard<std::mutex> lock(g_contexts_mutex);
+	uint64_t others = 0;
+	for(const fx_ctx* c = g_contexts; c; c = c->next)
+		if(c->device == ctx->device && c->touched > ctx->touched) others += ddf_bytes(c);
+	ctx->touched = ++g_touches;
+	const bool reread = ctx->reread;
+	ctx->reread = false;
+	const uint64_t row = (uint64_t)ctx->cfg.Nx * (ctx->cfg.storage == FX_FP32 ? 4u : 2u);
+	return steps == 1u && !reread && fx::crowds_cache(ddf_bytes(ctx), others, row) ? ctx->shape_sc_crowded : ctx->shape_sc;
+}
+
 uint32_t form_of(const fx::LaunchShape& s) {
 	return (s.cached ? FX_FORM_CACHED : 0u) | (s.pairs ? FX_FORM_TWO_CELLS : 0u) | (s.lin ? FX_FORM_LINEAR : 0u) | (s.xchunks ? FX_FORM_XCD_ROWS : 0u) |
 	       (s.buf ? FX_FORM_BUFFER : 0u) | (s.off32 ? FX_FORM_OFFSETS32 : 0u);
 }
-void launch_one_step(fx_ctx* ctx, const fx::LbmArgs& a) {
-	ctx->k->stream_collide(a, ctx->shape_sc, ctx->stream);
+void launch_one_step(fx_ctx* ctx, const fx::LbmArgs& a, const fx::LaunchShape& shape) {
+	ctx->k->stream_collide(a, shape, ctx->stream);
 	ctx->one_step++;
-	ctx->step_form = form_of(ctx->shape_sc);
+	ctx->step_form = form_of(shape);
 }
 void launch_two_steps(fx_ctx* ctx, const fx::LbmArgs& a, void* dst) {
 	ctx->k->two_steps(a, dst, ctx->shape_two, ctx->stream);
@@ -232,6 +260,7 @@ void launch_adjoint_step(fx_ctx* ctx, const fx::AdjointArgs& g) {
 // four steps each and leave the DDFs where they were; the rest, and all without a second
 // array, are single steps.
 void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps, void* second) {
+	const fx::LaunchShape& shape = step_shape(ctx, steps);
 	if(second) {
 		void* const fi = a.fi;
 		a.odd = (uint32_t)(t & 1ull);
@@ -245,7 +274,7 @@ void queue_steps(fx_ctx* ctx, fx::LbmArgs a, uint64_t t, uint64_t steps, void* s
 	}
 	for(; steps > 0u; steps--, t++) {
 		a.odd = (uint32_t)(t & 1ull);
-		launch_one_step(ctx, a);
+		launch_one_step(ctx, a, shape);
 	}
 }
 
@@ -659,6 +688,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	                                                                               : fx::stream_shape(cfg->Nx, cfg->Ny, cfg->Nz, true);
 	ctx->shape_uf.buf = N * cfg->velocity_set * eb <= 0xFFFFFFFFull;
 	ctx->shape_rec = ctx->shape_adj;
+	ctx->shape_sc_crowded = ctx->shape_sc;
 	const uint64_t ddf = N * cfg->velocity_set * eb;
 	if(ddf <= fx::CACHED_BYTES) {
 		if(ddf > fx::L2_BYTES && ctx->k->stream_collide_cached_pairs && fx::pair_rows(cfg->Nx) && fx::pair_extensions(cfg->storage, cfg->collision == FX_TRT, cfg->extensions)) {
@@ -670,8 +700,8 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 		if(ddf + 17u * N <= fx::CACHED_BYTES) ctx->shape_uf = fx::slab_shape(N); // the DDFs and what update_fields writes
 	}
 	ctx->shape_sc.alternate = N * cfg->velocity_set * eb >= fx::ALTERNATE_ORDER_BYTES;
-	ctx->shape_adj.alternate = ctx->shape_rec.alternate = ctx->shape_sc.alternate;
-	const uint32_t cap = ctx->shape_sc.cached ? 0u : ctx->k->stream_collide_waves_cap;
+	ctx->shape_sc_crowded.alternate = ctx->shape_adj.alternate = ctx->shape_rec.alternate = ctx->shape_sc.alternate;
+	const uint32_t cap = ctx->k->stream_collide_waves_cap;
 	hipError_t e = hipSetDevice(device);
 	if(e == hipSuccess) {
 		hipDeviceProp_t prop;
@@ -683,7 +713,8 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 			if(fx::two_steps_pay(two, cfg->Nx, cfg->Ny, cfg->Nz, cfg->velocity_set, cfg->collision == FX_TRT, cfg->extensions)) ctx->shape_two = two;
 		}
 		if(e == hipSuccess && cap)
-			ctx->shape_sc.lds = fx::occupancy_lds(cap, ctx->shape_sc.block.x, prop.maxSharedMemoryPerMultiProcessor, prop.sharedMemPerBlock);
+			for(fx::LaunchShape* s : {&ctx->shape_sc, &ctx->shape_sc_crowded})
+				if(!s->cached) s->lds = fx::occupancy_lds(cap, s->block.x, prop.maxSharedMemoryPerMultiProcessor, prop.sharedMemPerBlock);
 	}
 	if(e == hipSuccess) {
 		uint64_t free_b = 0;
@@ -708,6 +739,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 	}
 	{
 		std::lock_guard<std::mutex> lock(g_contexts_mutex);
+		ctx->touched = ++g_touches;
 		ctx->next = g_contexts;
 		g_contexts = ctx;
 	}
@@ -854,7 +886,7 @@ int fx_lbm_stream_collide(fx_ctx* ctx, void* fi, float* rho, float* u, const uin
 	const int rc = check_step_args(ctx, fi, rho, u, flags, F, alpha);
 	if(rc != FX_OK) return rc;
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	launch_one_step(ctx, make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha));
+	launch_one_step(ctx, make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), step_shape(ctx, 1u));
 	return check_launch("stream_collide");
 }
 
@@ -885,6 +917,7 @@ int fx_lbm_update_fields(fx_ctx* ctx, const void* fi, float* rho, float* u, cons
 	if(!rho || !u) return fail(FX_ERR_ARG, "rho and u must be device pointers");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
 	const fx::LbmArgs a = make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha);
+	touch(ctx, true);
 	ctx->k->update_fields(a, ctx->shape_uf, ctx->stream);
 	ctx->fields_form = form_of(ctx->shape_uf);
 	return check_launch("update_fields");
@@ -1038,6 +1071,7 @@ int fx_lbm_stream_collide_record(fx_ctx* ctx, void* fi, float* rho, float* u, co
 	if(ctx->cfg.extensions & (FX_MOVING_BOUNDARIES | FX_SUBGRID))
 		return fail(FX_ERR_CONFIG, "the adjoint does not differentiate MOVING_BOUNDARIES or SUBGRID");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
+	touch(ctx, false);
 	launch_record(ctx, make_args(ctx, fi, rho, u, flags, t, fx_, fy_, fz_, F, alpha), moments, fi);
 	return check_launch("stream_collide_record");
 }
@@ -1063,6 +1097,7 @@ int fx_lbm_adjoint_step(fx_ctx* ctx, float* lambda, const float* rho, const floa
 	if((ctx->cfg.extensions & FX_POROSITY) && !grad_alpha) return fail(FX_ERR_ARG, "POROSITY needs grad_alpha");
 	if((ctx->cfg.extensions & FX_EQUILIBRIUM_BOUNDARIES) && (!rho || !u)) return fail(FX_ERR_ARG, "TYPE_E presets rho/u required");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
+	touch(ctx, false);
 	launch_adjoint_step(ctx, adjoint_args(ctx, lambda, rho, u, flags, t, fx_, fy_, fz_, F, alpha, moments, plane_x, obj_weight, grad_alpha));
 	return check_launch("adjoint_step");
 }
@@ -1108,6 +1143,7 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 	// Before the window every span of steps runs from one checkpoint to the next or to the
 	// window: pairs of steps from the checkpoint, fi and work_fi (the backward sweep's) in turn, to
 	// the next checkpoint, so that no copy of the DDFs is made.
+	const fx::LaunchShape& shape = step_shape(ctx, 2u); // the objective goes over the DDFs too
 	void* now = fi; // the state of step t
 	for(uint64_t t = 0, n = 0; t < c.steps; t += n) {
 		void* const saved = adj->ckpt + (t / adj->k) * adj->fi_bytes;
@@ -1118,7 +1154,7 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 			a.odd = (uint32_t)(t & 1u);
 			ctx->k->objective_partial(a, c.plane_x, ctx->stream, partial + summed * adj->obj_blocks);
 			if(++summed == batch) sum_objective();
-			launch_one_step(ctx, a);
+			launch_one_step(ctx, a, shape);
 			n = 1u; // the objective looks at every step
 			continue;
 		}
@@ -1140,7 +1176,7 @@ int fx_lbm_forward(fx_ctx* ctx, fx_adjoint* adj, void* fi, float* rho, float* u,
 		}
 		for(uint64_t s = t + 2u * pairs; s < t + n; s++) {
 			a.odd = (uint32_t)(s & 1u);
-			launch_one_step(ctx, a);
+			launch_one_step(ctx, a, shape);
 		}
 	}
 	if(summed > 0u) sum_objective();
@@ -1175,6 +1211,7 @@ int fx_lbm_backward(fx_ctx* ctx, fx_adjoint* adj, const float* rho, const float*
 	const float wobj = (float)(1.0 / (double)(c.steps - c.window_begin));
 	fx::LbmArgs a = make_args(ctx, adj->work_fi, rho_w, u_w, flags, 0u, fx_, fy_, fz_, F, alpha);
 	a.ext &= ~FX_UPDATE_FIELDS; // the recomputation must not overwrite rho/u
+	touch(ctx, false);
 	for(uint64_t s = adj->checkpoints; s-- > 0u;) {
 		const uint64_t ts = s * adj->k, te = std::min<uint64_t>(c.steps, ts + adj->k);
 		for(uint64_t t = ts; t < te; t++) { // the first step from the checkpoint, which stays

@@ -56,6 +56,18 @@ inline LaunchShape linear_shape(uint64_t N, bool xcd) {
 // TRT FP16C (211 MiB) +2 %, D3Q19 170x168x168 to 184x180x180 (174 to 216 MiB) +23 to +56 %;
 // 128x192x192 D3Q27 (243 MiB) -6 to +40 %, 192^3 FP16S (256 MiB) -9 %, 256x256x128 -14 %.
 constexpr uint64_t CACHED_BYTES = 224ull << 20, L2_BYTES = 32ull << 20;
+// Whether a single step of a lattice of up to CACHED_BYTES, with `others` bytes of other lattices
+// gone over since its last one, takes the launch for DDFs from HBM.  Lattices stepped in turn, us per
+// step (with about 15 of host), cached -> that launch: D3Q19 SRT FP32 128^3 three lattices (456 MiB) 75.5 ->
+// 69.6, two (304) 66.5 -> 69.6; FP16S 128^3 seven (532) 49.6 -> 43.2, four (304) 46.9 -> 43.4,
+// three (228) 37.5 -> 43.1; D3Q27 TRT FP16C three (324) 59.5 -> 57.7; 256x96x64 -7 to -12 % in every
+// kernel, 160x120x100, 96x120x110 (16-bit rows on half lines) -13 to +2, 224x100x80 -9 to +4, 64^3 -3 to
+// +3.  Rows off half lines keep the cached launch, which has the better accesses for them:
+// 150x130x110 0 to +9 %, 201x75x99 0 to +18, 130x128x128 -5 to +6, 70^3 +1 to +4, 100x80x70 -1
+// to -5.  Runs of two steps and single steps followed by update_fields are as fast or faster
+// cached (0 to 10 %).
+constexpr uint64_t SHARED_CACHE_BYTES = 288ull << 20;
+inline bool crowds_cache(uint64_t own, uint64_t others, uint64_t row_bytes) { return own + others > SHARED_CACHE_BYTES && row_bytes % 64u == 0u; }
 inline LaunchShape slab_shape(uint64_t N) {
 	LaunchShape s = linear_shape(N, true);
 	s.cached = true;
