@@ -24,6 +24,7 @@ TYPE_I = 0x10
 TYPE_G = 0x20
 TYPE_X = 0x40
 TYPE_Y = 0x80
+STEPS_PER_CALL = 1000  # of LBM.run's calls (a multiple of four: pairs of launches of two steps)
 
 
 class Field:
@@ -183,10 +184,13 @@ class LBM:
                                                          self._ptr(self.F), self._ptr(self.porosity)))
                 self.ctx.sync()
                 self.t += 1
-        elif steps > 0:
-            check(self.ctx.lib.fx_lbm_run(*self._step_args(), self.t, steps, self.fx, self.fy, self.fz, self._ptr(self.F),
-                                          self._ptr(self.porosity), None))
-            self.t += steps
+        else:
+            end = self.t + steps
+            while self.t < end:  # Ctrl-C is seen, and t counts what was queued, between the calls
+                n = min(STEPS_PER_CALL, end - self.t)
+                check(self.ctx.lib.fx_lbm_run(*self._step_args(), self.t, n, self.fx, self.fy, self.fz, self._ptr(self.F),
+                                              self._ptr(self.porosity), None))
+                self.t += n
         if self.extensions & _abi.FX_UPDATE_FIELDS:
             self.t_last_update_fields = self.t
         self.ctx.sync()
