@@ -21,6 +21,14 @@ def oracle():
 
 
 @pytest.fixture(scope="session")
+def crowd():
+    from tests.crowd import Crowd
+    c = Crowd()
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="session")
 def refhelpers():
     """oracle/_ref/libref_helpers.so built from the reference's own host sources (skips where absent)."""
     import ctypes

@@ -30,7 +30,8 @@ def bits(names):
     return sum(EXT[n] for n in names)
 
 
-# 20x12x10: rows of one block; 300x4x3: rows of five 64-cell blocks (XCD-mapped grid)
+# 20x12x10: 12.8 rows per block; 300x4x3: rows longer than a block; both on slabs in the caches (the
+# kernels for arrays from HBM: tests/test_tiled_lattices.py)
 @pytest.mark.parametrize("grid", [(20, 12, 10), (300, 4, 3)], ids=lambda g: "x".join(map(str, g)))
 @pytest.mark.parametrize("q,collision", [(19, "SRT"), (19, "TRT"), (27, "SRT"), (27, "TRT")])
 @pytest.mark.parametrize("variant", ["porosity", "all", "clamped"])
@@ -119,7 +120,7 @@ def gpu_gradient(dims, rho, u, flags, alpha, steps, window, plane, k, fxv=1e-5):
     return J, g
 
 
-# 32x16x12: rows of one block; 260x8x6: rows of five 64-cell blocks (XCD-mapped grid)
+# 32x16x12: 8 rows per block; 260x8x6: rows longer than a block; both on slabs in the caches
 @pytest.mark.parametrize("grid", [(32, 16, 12), (260, 8, 6)], ids=lambda g: "x".join(map(str, g)))
 def test_gradient_matches_fp64_adjoint(oracle, grid):
     """Porous channel, 300 steps, objective over the last 100: checkpointed GPU gradient vs

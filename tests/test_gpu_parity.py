@@ -74,25 +74,35 @@ def compare_state(lbm, ref, oracle, storage, tag):
     assert bad.size == 0, f"{tag}: {bad.size} DDF values differ, first slot/cell {divmod(int(bad[0]), lbm.N)}: gpu {g[bad[0]]!r} oracle {o[bad[0]]!r}"
 
 
-# 20x12x10, 150x6x5, 520x3x3: rows off the 128-byte lines (cell-linear grid for 16-bit, and
-# for FP32 where Nx*4 misses them); 64x5x4: rows on lines, one block; 512x4x3: one block per
-# row, and two cells per lane for the D3Q19 16-bit kernels that take it; 1024x3x2: rows of
-# several blocks on the XCD-mapped grid, with both kernel forms
+# Lattices this small stay in the caches and run on slabs of the cell-linear grid, whatever Nx.
+# The kernels for DDFs from HBM run where another lattice crowds the cache (tests/crowd.py; rows
+# on half lines): 64x5x4: rows on lines, one block; 512x4x3: rows of two blocks (XCD-mapped
+# grid), one with two cells per lane for the D3Q19 16-bit kernels that take them; 1024x3x2: rows of several
+# blocks with both kernel forms.  (The other cell-linear kernels: tests/test_tiled_lattices.py.)
 GRIDS = {"20x12x10": (20, 12, 10), "150x6x5": (150, 6, 5), "520x3x3": (520, 3, 3), "64x5x4": (64, 5, 4), "512x4x3": (512, 4, 3),
          "1024x3x2": (1024, 3, 2)}
 
 
-@pytest.mark.parametrize("grid", GRIDS)
+CROWDED = ("64x5x4", "512x4x3", "1024x3x2")
+
+
+def step(lbm, crowd):
+    """One step, after one of the crowd if there is one."""
+    if crowd is None:
+        lbm.run(1)
+        assert lbm.ctx.launches().step_form & 2  # FX_FORM_CACHED
+    else:
+        crowd.run(lbm)
+
+
+@pytest.mark.parametrize("grid,crowded", [(g, False) for g in GRIDS] + [(g, True) for g in CROWDED])
 @pytest.mark.parametrize("q,collision,storage,ext", list(itertools.product((19, 27), ("SRT", "TRT"), ("FP32", "FP16S", "FP16C"), EXT_SETS)))
-def test_stream_collide_matches_oracle(oracle, q, collision, storage, ext, grid):
+def test_stream_collide_matches_oracle(oracle, crowd, q, collision, storage, ext, grid, crowded):
     """Random fields with scattered solids (and TYPE_E planes, forces, porosity): 7 steps,
-    both parities, ragged x-rows: Nx=20 in one 64-lane block; Nx=150, which with two cells
-    per lane leaves a block with a full wave, a partly live wave and dead second cells;
-    Nx=520, rows of several blocks on the 1-D XCD-mapped grid, whose last group of 8 rows
-    (9 rows here) is mostly padding.  These rows do not start on 128-byte lines, so the
-    kernels run on the cell-linear grid, whose blocks cross rows and planes (Nx=20: 12.8
-    rows per block); Nx=64 (one block per row) and Nx=512 (two blocks, XCD-mapped grid)
-    start every row on a line and keep the row grid."""
+    both parities, on slabs, whose blocks cross rows and planes (Nx=20: 12.8 rows per block)
+    and whose last block is partly live; crowded: on the row grid (Nx=64: one block per row),
+    the 1-D XCD-mapped grid (Nx=512: two blocks per row, 12 rows, so that the last group of 8 is
+    half padding; Nx=1024) and, for most D3Q19 16-bit kernels, two cells per lane (512, 1024)."""
     Nx, Ny, Nz = GRIDS[grid]
     names = EXT_SETS[ext]
     rho, u, flags = scenes.random_scene(Nx, Ny, Nz, seed=q + len(names), equilibrium_faces="EQUILIBRIUM_BOUNDARIES" in names)
@@ -112,7 +122,7 @@ def test_stream_collide_matches_oracle(oracle, q, collision, storage, ext, grid)
             lbm.flags.read_from_device()
             assert np.array_equal(lbm.flags.host, ref.flags) and (ref.flags & 3 == 3).any()
         for s in range(7):
-            lbm.run(1)
+            step(lbm, crowd if crowded else None)
             ref.step(1)
             compare_state(lbm, ref, oracle, storage, f"after step {s + 1}")
         lbm.u.read_from_device()
@@ -129,14 +139,16 @@ def test_stream_collide_matches_oracle(oracle, q, collision, storage, ext, grid)
 PAIR_SETS = {"equilibrium": ("EQUILIBRIUM_BOUNDARIES",), "porous": ("VOLUME_FORCE", "POROSITY", "PRECISE_DENSITY")}
 
 
+@pytest.mark.parametrize("crowded", [False, True])
 @pytest.mark.parametrize("collision,storage,ext", list(itertools.product(("SRT", "TRT"), ("FP16S", "FP16C"), PAIR_SETS)))
-def test_pair_kernel_dead_waves_and_lanes(oracle, collision, storage, ext):
+def test_pair_kernel_dead_waves_and_lanes(oracle, crowd, collision, storage, ext, crowded):
     """Two cells per lane (D3Q19 16-bit, rows of whole waves of 128 cells): rows whose first
     or last wave is all solid (the wave returns before its exchanges), rows with both cells
     of every fourth lane solid (the lane still passes codes between the x-shifted runs and
     the cells' lanes and writes its own back unchanged), scattered single solid cells and,
     with EQUILIBRIUM_BOUNDARIES, TYPE_E planes at the row ends, on 256x5x4 with rows of one
-    block; 6 steps, both parities, against the oracle."""
+    block; 6 steps, both parities, against the oracle.  Uncrowded, the same scene on slabs
+    with one cell per lane."""
     Nx, Ny, Nz = 256, 5, 4
     names = PAIR_SETS[ext]
     rho, u, flags = scenes.random_scene(Nx, Ny, Nz, seed=23, solid_fraction=0.05, equilibrium_faces="EQUILIBRIUM_BOUNDARIES" in names)
@@ -154,7 +166,9 @@ def test_pair_kernel_dead_waves_and_lanes(oracle, collision, storage, ext):
         lbm.initialize()
         ref.initialize()
         for s in range(6):
-            lbm.run(1)
+            step(lbm, crowd if crowded else None)
+            if crowded and (ext == "equilibrium" or collision == "TRT" or storage == "FP16C"):  # tune_pairs
+                assert lbm.ctx.launches().step_form & 4  # FX_FORM_TWO_CELLS
             ref.step(1)
             compare_state(lbm, ref, oracle, storage, f"after step {s + 1}")
         assert abs(lbm.mass() - ref.mass()) <= 1e-12 * abs(ref.mass())
@@ -221,9 +235,9 @@ def wide_codes(storage, rng, n):
 WIDE_SETS = {"plain": (), "volume_force": ("VOLUME_FORCE",), "drag": ("EQUILIBRIUM_BOUNDARIES", "FORCE_FIELD")}
 
 
-@pytest.mark.parametrize("grid", ["512x4x3", "20x12x10"])
+@pytest.mark.parametrize("grid,crowded", [("512x4x3", False), ("20x12x10", False), ("512x4x3", True), ("64x5x4", True)])
 @pytest.mark.parametrize("q,collision,storage,ext", list(itertools.product((19, 27), ("SRT", "TRT"), ("FP16S", "FP16C"), WIDE_SETS)))
-def test_codes_of_every_magnitude(oracle, q, collision, storage, ext, grid):
+def test_codes_of_every_magnitude(oracle, crowd, q, collision, storage, ext, grid, crowded):
     """One step from DDFs that are random 16-bit codes of every exponent: densities
     rho = 1 + sum f from below -1 to above 2, velocities j/rho of any size (clamped), outputs
     beyond the formats' range.  Planted cells load populations that give rho = 0 with j != 0
@@ -233,7 +247,8 @@ def test_codes_of_every_magnitude(oracle, q, collision, storage, ext, grid):
     densities 1e-30, 1e30 and 3e-20 (the 0.5/rho of the force block far outside the usual
     range).  Zero, non-finite and extreme densities take the division's general path where
     the kernels otherwise share one reciprocal of rho between u = j/rho and 0.5/rho.
-    Every code is compared with the oracle's."""
+    Every code is compared with the oracle's.  On slabs; crowded: with two cells per lane for the
+    D3Q19 kernels that take them, on the XCD-mapped grid (512) and the row grid (64)."""
     Nx, Ny, Nz = GRIDS[grid]
     N = Nx * Ny * Nz
     names = WIDE_SETS[ext]
@@ -287,7 +302,7 @@ def test_codes_of_every_magnitude(oracle, q, collision, storage, ext, grid):
         assert (dens[plant["zero"]] == 0).all() and (dens[plant["tiny"]] > 0).all() and (dens[plant["tiny"]] < 1e-7).all()
         assert (dens[plant["negative"]] == -2.0 ** -8).all() and (dens[plant["ones"]] == 2.0 - 2.0 ** -23).all()
         assert dens[fluid].min() < -1 and dens[fluid].max() > 2
-        lbm.run(1)
+        step(lbm, crowd if crowded else None)
         ref.step(1)
         compare_state(lbm, ref, oracle, storage, "after one step")
     finally:
@@ -350,16 +365,15 @@ def test_full_size_256_two_steps(oracle):
 def test_lattice_beyond_4_gib_matches_its_tile(storage, reps, q, collision, ext, n0):
     """64-bit addressing at full scale: a 512x512x256 FP32 / 512^3 FP16S D3Q19 SRT lattice
     (5.1 GB of DDFs, slot offsets up to 4.8 GB; FP32 above 4 GiB on the cell-linear grid,
-    FP16S on the XCD-mapped row grid, the 64^3 lattices on the row grid) filled with a
-    Taylor-Green vortex of period 64 is the 64^3 vortex repeated, so after 3 steps every
-    64^3 tile of slots 0, 9, 17 and 18 (and 26 for D3Q27) equals the 64^3 lattice's DDFs bit
-    for bit (the 64^3 lattice is oracle-checked above).  The D3Q27 TRT FP16C kernel with
-    EQUILIBRIUM_BOUNDARIES + FORCE_FIELD (no TYPE_E cells, zero force field) takes buffer
-    instructions at 64^3 and, with 5.4 GB of DDFs at 512x512x384, 32-bit slot offsets; the
-    D3Q19 TRT FP16C two-cells-per-lane kernel takes buffer instructions at 64^3 and global
-    addressing with 4.5 GB at 512x512x448; the 20^3 vortex (cell-linear grid, rows off the
-    lines) tiled to 500x500x460 (4.4 GB of FP16S DDFs) leaves the cell-linear grid's buffer
-    instructions for its 32-bit slot offsets.  Every large lattice here also takes its
+    FP16S on the XCD-mapped row grid, the 64^3 lattices on slabs in the caches) filled with a
+    Taylor-Green vortex of period 64 is the 64^3 vortex repeated, so after 3 single steps and
+    4 more (FP32: two launches of two steps) every 64^3 tile of slots 0, 9, 17 and 18 (and 26 for
+    D3Q27) equals the 64^3 lattice's DDFs bit for bit (the 64^3 lattice is oracle-checked above).  The D3Q27 TRT FP16C kernel with
+    EQUILIBRIUM_BOUNDARIES + FORCE_FIELD (no TYPE_E cells, zero force field) takes, with 5.4 GB
+    of DDFs at 512x512x384, 32-bit slot offsets; the D3Q19 TRT FP16C two-cells-per-lane kernel
+    takes global addressing with 4.5 GB at 512x512x448; the 20^3 vortex (rows off the lines)
+    tiled to 500x500x460 (4.4 GB of FP16S DDFs) takes the cell-linear grid's 32-bit slot
+    offsets in place of its buffer instructions.  Every large lattice here also takes its
     blocks in reverse order on odd steps."""
     import fluidx3d_amd as fx
     rho0, u0, _ = scenes.taylor_green(n0, n0, n0)
@@ -368,19 +382,22 @@ def test_lattice_beyond_4_gib_matches_its_tile(storage, reps, q, collision, ext,
     big = fx.LBM(n0 * reps[2], n0 * reps[1], n0 * reps[0], 1.0 / 6.0, **opts)
     try:
         small.rho.host[:] = rho0; small.u.host[:] = u0
-        small.run(3)
-        ref = small.read_ddfs().reshape(q, n0, n0, n0)
+        small.initialize()
         big.rho.host[:] = np.tile(rho0.reshape(n0, n0, n0), reps).ravel()
         for d in range(3):
             big.u.host[d * big.N:(d + 1) * big.N] = np.tile(u0[d * n0 ** 3:(d + 1) * n0 ** 3].reshape(n0, n0, n0), reps).ravel()
-        big.run(3)
         esize = 4 if storage == "FP32" else 2
         assert q * big.N * esize > 4 << 30
-        for i in (0, 9, 17, 18) + ((26,) if q == 27 else ()):
-            slot = np.empty(big.N, np.float32 if storage == "FP32" else np.uint16)
-            big.ctx.read(big.fi, slot, offset=i * big.N * esize)
-            tiles = slot.reshape(reps[0], n0, reps[1], n0, reps[2], n0)
-            assert np.array_equal(tiles, np.broadcast_to(ref[i][None, :, None, :, None, :], tiles.shape)), f"slot {i}"
+        for steps in (3, 4):
+            small.run(steps)
+            ref = small.read_ddfs().reshape(q, n0, n0, n0)
+            big.run(steps)
+            assert big.ctx.launches().two_steps == (2 if storage == "FP32" and steps == 4 else 0)
+            for i in (0, 9, 17, 18) + ((26,) if q == 27 else ()):
+                slot = np.empty(big.N, np.float32 if storage == "FP32" else np.uint16)
+                big.ctx.read(big.fi, slot, offset=i * big.N * esize)
+                tiles = slot.reshape(reps[0], n0, reps[1], n0, reps[2], n0)
+                assert np.array_equal(tiles, np.broadcast_to(ref[i][None, :, None, :, None, :], tiles.shape)), (steps, f"slot {i}")
     finally:
         small.close()
         big.close()

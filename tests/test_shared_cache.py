@@ -6,17 +6,9 @@ import numpy as np
 import pytest
 
 from tests import scenes
-from tests.crowd import Crowd
 from tests.test_gpu_parity import compare_state, setup_pair
 
 pytestmark = pytest.mark.gpu
-
-
-@pytest.fixture(scope="module")
-def crowd():
-    c = Crowd()
-    yield c
-    c.close()
 
 
 def cached(lbm):
