@@ -100,3 +100,54 @@ def test_allocation_is_outside_the_timed_region():
             lbm.close()
     print("first", [round(v) for v in first], "later", [round(v) for v in later])
     assert min(first) < 1.5 * min(later), (first, later)
+
+
+def test_threads():
+    """Lattices run by one thread each while another thread declines and allows their second
+    arrays and creates and destroys contexts: the bits of single steps."""
+    import threading
+    import fluidx3d_amd as fx
+    lbms = [scene_lbm(fx, SIZE, 19, "SRT", ()) for _ in range(3)]
+    ref = scene_lbm(fx, SIZE, 19, "SRT", ())
+    errors, done = [], threading.Event()
+
+    def guarded(f):
+        def g(*args):
+            try:
+                f(*args)
+            except Exception as e:  # noqa: BLE001
+                errors.append(e)
+        return g
+
+    @guarded
+    def work(lbm):
+        for steps in (4, 7, 8, 1, 12) * 4:
+            lbm.run(steps)
+
+    @guarded
+    def disturb():
+        k = 0
+        while not done.is_set():
+            lbms[k % 3].set_second_array(k % 2 == 1)
+            other = fx.LBM(64, 32, 32, 0.05)
+            other.run(2)
+            other.close()
+            k += 1
+
+    try:
+        threads = [threading.Thread(target=work, args=(lbm,)) for lbm in lbms]
+        extra = threading.Thread(target=disturb)
+        for th in threads + [extra]:
+            th.start()
+        for th in threads:
+            th.join()
+        done.set()
+        extra.join()
+        assert not errors, errors
+        single_steps(ref, lbms[0].t)
+        want = ref.read_ddfs().view(np.uint32)
+        for lbm in lbms:
+            assert lbm.t == 128 and np.array_equal(lbm.read_ddfs().view(np.uint32), want)
+    finally:
+        for lbm in lbms + [ref]:
+            lbm.close()

@@ -85,12 +85,12 @@ def test_rule(lines):
 
 POROUS = ("VOLUME_FORCE", "POROSITY", "PRECISE_DENSITY")
 EQ_FF = ("EQUILIBRIUM_BOUNDARIES", "FORCE_FIELD")
-# (size, q, collision, extensions): every kernel, on lattices that the rule takes
+# (size, q, collision, extensions): every kernel, on lattices that the rule takes but for one
 CASES = [
     ((128, 61, 58), 19, "SRT", ()),              # one tile across, clipped in y and z
     ((64, 143, 51), 19, "SRT", ()),              # 64-wide tiles
     ((50, 143, 63), 19, "SRT", ()),              # 14 lanes idle
-    ((257, 81, 34), 19, "SRT", ()),              # three tiles across, the last of 65 cells
+    ((321, 81, 34), 19, "SRT", ()),              # three tiles across, the last of 65 cells
     ((350, 81, 82), 19, "SRT", ()),              # 91 %, one array of two in the caches
     ((300, 2, 800), 19, "SRT", ()),              # rows 0 and 1 are each other's neighbours twice
     ((300, 400, 4), 19, "SRT", ()),
@@ -114,6 +114,40 @@ CASES = [
     ((100, 63, 57), 27, "SRT", ("MOVING_BOUNDARIES", "FORCE_FIELD", "EQUILIBRIUM_BOUNDARIES")),
     ((128, 191, 97), 27, "TRT", ("MOVING_BOUNDARIES", "SUBGRID")),
 ]
+SINGLE_STEPS = [((129, 64, 60), 27, "SRT", ())]
+
+
+def test_rule_of_the_cases(tmp_path):
+    """two_steps_pay takes every lattice of CASES but SINGLE_STEPS, and the kernel subsets that have
+    a k_two_steps are all FP32 ones but the one with every extension."""
+    bits = {"VOLUME_FORCE": 1, "FORCE_FIELD": 2, "EQUILIBRIUM_BOUNDARIES": 4, "POROSITY": 16, "PRECISE_DENSITY": 32, "MOVING_BOUNDARIES": 64, "SUBGRID": 128}
+    rows = "".join("{%d,%d,%d,%d,%d,%d}," % (*size, q, collision == "TRT", sum(bits[e] for e in ext)) for size, q, collision, ext in CASES)
+    program = r'''
+#include "lbm_launch.hpp"
+#include <cstdio>
+using namespace fx;
+template<int Q, bool TRT, uint32_t EXT> void tune() {
+  printf("%d%d%d ", (int)tune_two_steps(Q, ST_FP32, TRT, EXT), (int)tune_two_steps(Q, ST_FP16S, TRT, EXT), (int)tune_two_steps(Q, ST_FP16C, TRT, EXT));
+}
+template<uint32_t EXT> void tune_all() { tune<19, false, EXT>(); tune<19, true, EXT>(); tune<27, false, EXT>(); tune<27, true, EXT>(); }
+int main() {
+  constexpr uint32_t E = EXT_EQUILIBRIUM_BOUNDARIES, FF = EXT_FORCE_FIELD, VF = EXT_VOLUME_FORCE, POROUS = VF | EXT_POROSITY | EXT_PRECISE_DENSITY;
+  tune_all<0u>(); tune_all<E>(); tune_all<VF>(); tune_all<E | FF>(); tune_all<POROUS>(); tune_all<EXT_LES>(); tune_all<EXT_LES_MOVING>();
+  printf("\n");
+  tune_all<EXT_ALL>();
+  printf("\n");
+  const unsigned cases[][6] = {ROWS};
+  for (const auto& c : cases) printf("%d", (int)two_steps_pay(two_step_shape(c[0], c[1], c[2], 256), c[0], c[1], c[2], c[3], c[4], c[5]));
+  return 0;
+}
+'''.replace("ROWS", rows)
+    src, exe = tmp_path / "p.hip", tmp_path / "p"
+    src.write_text(program)
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-host-only", "-O1", "-std=c++17", "-I" + os.path.join(ROOT, "fluidx3d_amd", "csrc"),
+                    "-I" + os.path.join(ROOT, "include"), str(src), "-o", str(exe)], check=True, capture_output=True, text=True)
+    subsets, everything, taken = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines()
+    assert set(subsets.split()) == {"100"} and set(everything.split()) == {"000"}
+    assert taken == "".join("0" if c in SINGLE_STEPS else "1" for c in CASES)
 
 
 def scene_lbm(fx, size, q, collision, extensions, nu=0.03):
@@ -142,9 +176,14 @@ def single_steps(lbm, steps):
 def test_run_equals_single_steps(size, q, collision, extensions):
     import fluidx3d_amd as fx
     a, b = (scene_lbm(fx, size, q, collision, extensions) for _ in range(2))
+    takes = (size, q, collision, extensions) not in SINGLE_STEPS
     try:
         for steps in (4, 1, 7, 10):  # from even and odd t; 0, 1, 3 and 2 single steps after the pairs
+            before = a.ctx.launches()
             a.run(steps)
+            after = a.ctx.launches()
+            two = steps // 4 * 2 if takes else 0
+            assert (after.two_steps - before.two_steps, after.one_step - before.one_step) == (two, steps - 2 * two)
             single_steps(b, steps)
             x, y = a.read_ddfs(), b.read_ddfs()
             same = x.view(np.uint32) == y.view(np.uint32)
@@ -166,6 +205,7 @@ def test_run_equals_oracle(oracle):
         ref.initialize()
         lbm.run(9)
         ref.step(9)
+        assert lbm.ctx.launches().two_steps == 4
         assert np.array_equal(lbm.read_ddfs(), ref.fi)
     finally:
         lbm.close()
@@ -186,6 +226,8 @@ def test_adjoint_equals_single_steps(interval, window):
         lbm.rho.host[:], lbm.u.host[:], lbm.flags.host[:], lbm.porosity.host[:] = rho, u, flags, alpha
         adj = Adjoint(lbm, steps=31, window_begin=window, plane_x=127, checkpoint_interval=k)
         states.append((adj.forward(), lbm.read_ddfs(), adj.backward(), adj.backward()))
+        spans = [min(k - t % k, window - t) for t in range(0, window, k)]
+        assert lbm.ctx.launches().two_steps == sum(n // 2 for n in spans)
         adj.close()
         lbm.close()
     (J, f, g, again), (J1, f1, g1, _) = states
