@@ -394,7 +394,7 @@ __global__ __launch_bounds__(RED_BLOCK) void k_object_partial(const float* F, co
 	};
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const uint64_t step = (uint64_t)gridDim.x * RED_BLOCK * 4u; // 256 cells per wave
-	for(uint64_t c0 = ((uint64_t)blockIdx.x * (RED_BLOCK / 64) + wave) * SCAN_CELLS; c0 < N; c0 += step) scan_flags(flags, N, c0, 0xFFu, marker, add);
+	for(uint64_t c0 = ((uint64_t)blockIdx.x * (RED_BLOCK / 64) + wave) * SCAN_CELLS; c0 < N; c0 += step) scan_flags(flags, N, c0, marker, add);
 	for(int k = 0; k < 4; k++) red[k][threadIdx.x] = acc[k];
 	__syncthreads();
 	for(int s = RED_BLOCK / 2; s > 0; s >>= 1) {

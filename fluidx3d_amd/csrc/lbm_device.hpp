@@ -32,7 +32,6 @@ constexpr float DEF_C = 0.57735027f; // lattice speed of sound, src/lbm.cpp:366
 constexpr float THIRD = 0.33333334f; // src/kernel.cpp:1093-1099
 constexpr float SMAGORINSKY = 0.76421222f; // 18*sqrt(2)*(C*Delta)^2, src/kernel.cpp:1591
 
-// Kernel arguments, passed by value (kernarg segment -> scalar registers).
 // n / d for n below 2^31 and d from 1 to 2^31 as a multiplication (Granlund and Montgomery, "Division
 // by invariant integers using multiplication", 1994): m = ceil(2^(31+l) / d) fits 32 bits for
 // l = ceil(log2 d), and n * (m*d - 2^(31+l)) < 2^(31+l).
@@ -47,6 +46,7 @@ struct Divisor {
 	}
 	__host__ __device__ uint32_t quotient(uint32_t n) const { return m ? (uint32_t)(((uint64_t)n * m) >> 32) >> shift : n; }
 };
+// Kernel arguments, passed by value (kernarg segment -> scalar registers).
 struct LbmArgs {
 	void* fi;
 	float* rho;
@@ -987,9 +987,11 @@ template<bool XCD> __device__ __forceinline__ bool block_coords(const LbmArgs& a
 	y = row - z * a.Ny;
 	return true;
 }
-// Segment of block L where each XCD takes one eighth of the lattice, a slab of consecutive
+// Segment of block L where each XCD takes one eighth of the grid, a slab of consecutive
 // segments (blocks: a multiple of 8), so that the lines a step leaves in an L2 are the ones
-// that its XCD reads in the next step, except at the slabs' ends.  A permutation.
+// that its XCD reads in the next step, except at the slabs' ends.  A permutation.  The grid is
+// padded to whole groups of 64 blocks (linear_blocks), so the last XCDs' slabs of a small lattice
+// are padding: 24x16x12 (18 blocks) runs on three XCDs, 65 blocks on five, 393 and more on all.
 __host__ __device__ inline uint64_t slab_segment(uint64_t L, uint64_t blocks) { return (L & 7u) * (blocks >> 3) + (L >> 3); }
 // Segment (block of consecutive cells) of block L on the cell-linear grid.  The hardware
 // hands consecutive blocks to the 8 XCDs in turn; with xcd and a grid of whole groups of
@@ -1312,17 +1314,17 @@ __global__ __launch_bounds__(BLOCK) void k_update_fields(LbmArgs a) {
 	}
 }
 
-// f(n) for the cells n of [c0, c0 + 256) whose flags & mask equal value, each on one lane of a
+// f(n) for the cells n of [c0, c0 + 256) whose flags equal value, each on one lane of a
 // wave (all 64 lanes call it): every lane reads four flags at once, and the runs of 64 cells
 // that hold a match are then taken one cell per lane, so what f reads is consecutive.
 constexpr uint32_t SCAN_CELLS = 256u;
-template<class F> __device__ __forceinline__ void scan_flags(const uint8_t* flags, uint64_t N, uint64_t c0, uint32_t mask, uint32_t value, F&& f) {
+template<class F> __device__ __forceinline__ void scan_flags(const uint8_t* flags, uint64_t N, uint64_t c0, uint32_t value, F&& f) {
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint64_t mine = c0 + lane * 4u;
 	uint32_t word = (value ^ 0xFFu) * 0x01010101u; // matches nothing
 	if(mine + 4u <= N && ((uint64_t)flags & 3u) == 0u) word = *(const uint32_t*)(flags + mine);
 	else for(uint32_t j = 0; j < 4u; j++) if(mine + j < N) word = (word & ~(0xFFu << (8u * j))) | ((uint32_t)flags[mine + j] << (8u * j));
-	const uint32_t t = (word & (mask * 0x01010101u)) ^ (value * 0x01010101u); // a zero byte: a match
+	const uint32_t t = word ^ (value * 0x01010101u); // a zero byte: a match
 	uint64_t lanes = __ballot(((t - 0x01010101u) & ~t & 0x80808080u) != 0u); // lanes 16r .. 16r+15: run r
 	while(lanes) {
 		const uint32_t run = (uint32_t)__builtin_ctzll(lanes) >> 4;

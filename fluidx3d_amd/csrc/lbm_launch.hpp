@@ -44,7 +44,7 @@ inline LaunchShape linear_shape(uint64_t N, bool xcd) {
 	return s;
 }
 // Lattices whose DDFs stay in the last-level cache (256 MiB) from one step to the next: no
-// non-temporal accesses, which leave the lines out of it, and one slab of the lattice per XCD
+// non-temporal accesses, which leave the lines out of it, and one slab of the grid per XCD
 // (slab_segment; slab_shape, the cell-linear grid whether rows start on lines or not).  Bound
 // by that cache (7.0 TB/s in place, against 6.3 from HBM) and below L2_BYTES, all L2s together, by
 // the start of a launch.  fx_lbm_run, us per step before -> now: D3Q19 SRT FP16S 64^3 7.8 ->

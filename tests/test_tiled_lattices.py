@@ -265,6 +265,12 @@ int main() {
     if (s.grid.x % 8u || (uint64_t)s.grid.x * s.block.x < N || !s.cached || !s.lin) bad++;
     for (uint64_t L = 0; L < s.grid.x; L++) { const uint64_t g = slab_segment(L, s.grid.x); if (g >= s.grid.x || seen[g]++ || g / (s.grid.x / 8u) != L % 8u) bad++; }
   }
+  for (uint64_t b = 1; b < 1000; b++) { // XCDs with blocks of the lattice, not only padding (slab_segment's comment)
+    const LaunchShape s = slab_shape(b * 256);
+    unsigned used = 0;
+    for (uint64_t xcd = 0; xcd < 8; xcd++) used += slab_segment(xcd, s.grid.x) < b;
+    if ((b == 18 && used != 3) || (b == 65 && used != 5) || (b == 392 && used == 8) || (b > 392 && used != 8)) bad++;
+  }
   printf("bad %u\n", bad);
   return 0;
 }
@@ -273,7 +279,7 @@ int main() {
 
 def test_cell_of_a_block(tmp_path):
     """Division by multiplication (Divisor) below 2^31, and the slabs of slab_segment: each
-    segment once, an eighth of them per XCD."""
+    segment of the padded grid once, an eighth of them per XCD."""
     src, exe = tmp_path / "p.hip", tmp_path / "p"
     src.write_text(PROGRAM)
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
