@@ -121,14 +121,17 @@ uint64_t ddf_bytes(const fx_ctx* ctx) {
 // ---- second DDF arrays ----
 // two_steps launches read one DDF array and write another.  The second one belongs to the
 // context that runs them and is allocated by its first run that can use it, if there is room
-// (second_array_fits) and the caller did not decline it (fx_ctx_second_array); it is
-// kept for the next run, and given back when the caller asks for that, when any context of the
-// device cannot allocate what its caller asked for (allocate_device), or with the context.  Launches on one context's stream run in order, so the next call may use the
-// array while the last one's launches still run; a call from another thread that comes while
-// one is queueing takes single steps.  g_contexts_mutex guards the list of contexts (linked
-// through the contexts, so that a run allocates no host memory and cannot throw) and every
-// context's `second`, `second_busy`, `second_allowed`, `touched` and `reread`.
-std::mutex g_contexts_mutex;
+// (second_array_fits) and the caller did not decline it (fx_ctx_second_array); it is kept for the
+// next run, and given back when the caller asks for that, when any context of the device cannot
+// allocate what its caller asked for (allocate_device), or with the context.  Launches on one
+// context's stream run in order, so the next call may use the array while the last one's
+// launches still run; a call from another thread that comes while one is queueing takes single
+// steps.
+// Contexts are linked in a list, so that a run allocates no host memory and cannot throw.
+// g_second_mutex guards every context's `second`, `second_busy` and `second_allowed`, and may be
+// held over allocations and waits; g_contexts_mutex guards `touched`, `reread` and g_touches, and
+// is taken by every step.  The list changes with both held (g_second_mutex first).
+std::mutex g_second_mutex, g_contexts_mutex;
 fx_ctx* g_contexts = nullptr;
 
 // Allocations must not disturb a stream capture that another library has open in this thread.
@@ -147,7 +150,7 @@ void release_second_locked(fx_ctx* ctx) {
 }
 // Gives back every second array of the device that no call is using; true if there was one.
 bool release_second_arrays(int device) {
-	std::lock_guard<std::mutex> lock(g_contexts_mutex);
+	std::lock_guard<std::mutex> lock(g_second_mutex);
 	bool any = false;
 	for(fx_ctx* c = g_contexts; c; c = c->next)
 		if(c->device == device && c->second && !c->second_busy) { release_second_locked(c); any = true; }
@@ -186,7 +189,7 @@ struct SecondArray {
 	void* array = nullptr;
 	SecondArray(fx_ctx* c, bool wanted) : ctx(c) {
 		if(!wanted) return;
-		std::lock_guard<std::mutex> lock(g_contexts_mutex);
+		std::lock_guard<std::mutex> lock(g_second_mutex);
 		if(!ctx->second_allowed || ctx->second_busy) return; // busy: another thread is queueing launches on it
 		if(!ctx->second) {
 			const RelaxedCapture relaxed;
@@ -199,7 +202,7 @@ struct SecondArray {
 	}
 	~SecondArray() {
 		if(!array) return;
-		std::lock_guard<std::mutex> lock(g_contexts_mutex);
+		std::lock_guard<std::mutex> lock(g_second_mutex);
 		ctx->second_busy = false;
 		if(!ctx->second_allowed) release_second_locked(ctx); // declined in the meantime
 	}
@@ -738,7 +741,7 @@ int fx_ctx_create(int device, const fx_lbm_config* cfg, fx_ctx** out) {
 		return fail(FX_ERR_HIP, msg);
 	}
 	{
-		std::lock_guard<std::mutex> lock(g_contexts_mutex);
+		std::lock_guard<std::mutex> second(g_second_mutex), lock(g_contexts_mutex);
 		ctx->touched = ++g_touches;
 		ctx->next = g_contexts;
 		g_contexts = ctx;
@@ -752,10 +755,10 @@ int fx_ctx_destroy(fx_ctx* ctx) {
 	(void)hipSetDevice(ctx->device);
 	if(ctx->stream) (void)hipStreamSynchronize(ctx->stream);
 	{
-		std::lock_guard<std::mutex> lock(g_contexts_mutex);
-		release_second_locked(ctx);
+		std::lock_guard<std::mutex> second(g_second_mutex), lock(g_contexts_mutex);
 		for(fx_ctx** c = &g_contexts; *c; c = &(*c)->next) if(*c == ctx) { *c = ctx->next; break; }
 	}
+	if(ctx->second) (void)hipFree(ctx->second);
 	for(void* p : ctx->buffers) (void)hipFree(p);
 	if(ctx->partial) (void)hipFree(ctx->partial);
 	if(ctx->result) (void)hipFree(ctx->result);
@@ -782,15 +785,21 @@ int fx_ctx_launches(const fx_ctx* ctx, fx_launches* out) {
 int fx_ctx_second_array(fx_ctx* ctx, int allowed) {
 	if(!ctx) return fail(FX_ERR_ARG, "null context");
 	if(set_device(ctx) != FX_OK) return FX_ERR_HIP;
-	std::lock_guard<std::mutex> lock(g_contexts_mutex);
-	ctx->second_allowed = allowed != 0;
-	if(!allowed && !ctx->second_busy) release_second_locked(ctx); // busy: that call gives it back (SecondArray)
+	{
+		std::lock_guard<std::mutex> lock(g_second_mutex);
+		ctx->second_allowed = allowed != 0;
+	}
+	if(!allowed) {
+		(void)hipStreamSynchronize(ctx->stream); // the long wait, without the lock
+		std::lock_guard<std::mutex> lock(g_second_mutex);
+		if(!ctx->second_allowed && !ctx->second_busy) release_second_locked(ctx); // busy: that call gives it back (SecondArray)
+	}
 	return FX_OK;
 }
 
 int fx_ctx_second_array_bytes(const fx_ctx* ctx, uint64_t* held, uint64_t* most) {
 	if(!ctx) return fail(FX_ERR_ARG, "null context");
-	std::lock_guard<std::mutex> lock(g_contexts_mutex);
+	std::lock_guard<std::mutex> lock(g_second_mutex);
 	if(held) *held = ctx->second ? ddf_bytes(ctx) : 0u;
 	if(most) *most = ctx->shape_two.grid ? ddf_bytes(ctx) : 0u;
 	return FX_OK;

@@ -151,3 +151,33 @@ def test_threads():
     finally:
         for lbm in lbms + [ref]:
             lbm.close()
+
+
+def test_returning_it_does_not_hold_up_other_contexts():
+    """Giving a second array back waits for its context's work; steps of other contexts are queued
+    meanwhile.  (One lock for both held the calls up for the whole wait, about 200 ms here.)"""
+    import threading
+    import time
+    import fluidx3d_amd as fx
+    from fluidx3d_amd._abi import check
+    busy, other = fx.LBM(256, 256, 256, 0.05), fx.LBM(64, 32, 32, 0.05)
+    try:
+        busy.run(4)
+        other.run(4)
+        other.update_fields()
+        check(busy.ctx.lib.fx_lbm_run(*busy._step_args(), busy.t, 800, 0.0, 0.0, 0.0, None, None, None))
+        waiting = []
+        th = threading.Thread(target=lambda: waiting.append((busy.set_second_array(False), time.perf_counter())[1]))
+        t0 = time.perf_counter()
+        th.start()
+        time.sleep(0.02)
+        t1 = time.perf_counter()
+        check(other.ctx.lib.fx_lbm_stream_collide(*other._step_args(), other.t, 0.0, 0.0, 0.0, None, None))
+        t2 = time.perf_counter()
+        th.join()
+        print(f"given back after {1e3 * (waiting[0] - t0):.0f} ms, step queued in {1e3 * (t2 - t1):.2f} ms")
+        assert waiting[0] - t0 > 0.1 and t2 - t1 < 0.05
+        assert busy.ctx.second_array_bytes()[0] == 0
+    finally:
+        busy.close()
+        other.close()
