@@ -241,13 +241,13 @@ uint32_t form_of(const fx::LaunchShape& s) {
 }
 void launch_one_step(fx_ctx* ctx, const fx::LbmArgs& a, const fx::LaunchShape& shape) {
 	ctx->k->stream_collide(a, shape, ctx->stream);
-	ctx->one_step++;
-	ctx->step_form = form_of(shape);
+	ctx->one_step.fetch_add(1u, std::memory_order_relaxed);
+	ctx->step_form.store(form_of(shape), std::memory_order_relaxed);
 }
 void launch_two_steps(fx_ctx* ctx, const fx::LbmArgs& a, void* dst) {
 	ctx->k->two_steps(a, dst, ctx->shape_two, ctx->stream);
-	ctx->two_steps++;
-	ctx->step_form = FX_FORM_TWO_STEPS | (ctx->shape_two.cached ? FX_FORM_CACHED : 0u);
+	ctx->two_steps.fetch_add(1u, std::memory_order_relaxed);
+	ctx->step_form.store(FX_FORM_TWO_STEPS | (ctx->shape_two.cached ? FX_FORM_CACHED : 0u), std::memory_order_relaxed);
 }
 
 void launch_record(fx_ctx* ctx, const fx::LbmArgs& a, float* moments, void* dst) {
